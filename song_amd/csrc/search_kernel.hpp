@@ -21,12 +21,11 @@
 //   visited  : H slots, no deletion: compact 16-bit entries in groups of 8 (vis16_insert) or
 //              32-bit (id + 1) in groups of 4 (vis_insert), one 16-byte read per group; or,
 //              approximate, a blocked Bloom filter of 2^hlog 32-bit words (bloom_insert)
-//   scratch  : 64 keys    merge staging of the queue head (the head itself is one key per
-//                          lane in registers, ascending over lanes [h, h + nq), nq <= 64)
 //   best     : pq keys, sorted ascending, first nbest live (pq-best expanded list); absent
 //              with bglob, where the list's front lives in the wave slot's global region
 //   cid      : 256 u32   candidate ids of the current expansion / radix-select bins
 //   qv       : qld f32   the query, zero-padded to a multiple of 16
+// The queue head is one key per lane in registers, ascending over lanes [h, h + nq), nq <= 64.
 // The bag (qcap = pq + slack + 128 keys, unsorted, first bn live) is in global memory, one
 // region per wave slot: it is written by plain stores as candidates arrive and read only when
 // the head runs empty or the bag nears its capacity, so LDS holds only what every step
@@ -204,6 +203,22 @@ template <> struct KeySel<true> { using T = KeyD; };
 // ---------------------------------------------------------------- wave helpers
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63u); }
+// The lane index as a value the compiler cannot see through, for the rare paths (refill,
+// truncation, front insert): their lane masks -- (lane & j) == 0 of every bitonic step, lane < n of
+// every block -- are then computed where they are used.  From the plain lane index they are loop
+// invariants, which the compiler hoists out of the expansion loop into scalar register pairs; the
+// loop has about 100 scalar registers, so 130-250 of them were spilled to vector lanes and read back
+// on the common path.
+__device__ __forceinline__ int rare_lane() {
+    int l = lane_id();
+    asm volatile("" : "+v"(l));
+    return l;
+}
+// a wave-uniform 64-bit mask as a per-lane predicate (the mask is used as the condition register
+// as it is: no shift or compare per lane)
+__device__ __forceinline__ bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+// the lowest n bits, n in [0, 64]
+__device__ __forceinline__ uint64_t low_bits(int n) { return n >= 64 ? ~0ull : (1ull << n) - 1ull; }
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 __device__ __forceinline__ int lanes_below(uint64_t m) {
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -292,10 +307,12 @@ __device__ __forceinline__ uint32_t zero_halves(uint32_t x) { return (x - 0x0001
 __device__ __forceinline__ bool group_has(const uint4 &v, uint32_t ee) {
     return (zero_halves(v.x ^ ee) | zero_halves(v.y ^ ee) | zero_halves(v.z ^ ee) | zero_halves(v.w ^ ee)) != 0u;
 }
-// 0: present, 1: inserted, 2: no room within 4 groups
-__device__ __forceinline__ int vis16_insert(uint32_t *vis, int gbits, int idbits, uint32_t id) {
-    uint32_t home, lo1;
-    vis16_key(id, idbits, gbits, home, lo1);
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_min16(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+// 0: present, 1: inserted, 2: no room within 4 groups; every group from displacement d0 on
+__device__ __forceinline__ int vis16_probe(uint32_t *vis, int gbits, uint32_t home, uint32_t lo1) {
     const uint32_t gmask = (1u << gbits) - 1u;
     for (uint32_t d = 0; d < 4u; ++d) {
         const uint32_t g = (home + d) & gmask;
@@ -315,6 +332,31 @@ __device__ __forceinline__ int vis16_insert(uint32_t *vis, int gbits, int idbits
         }
     }
     return 2;
+}
+// 0: present, 1: inserted, 2: no room within 4 groups.  The home group decides almost every id, so
+// it is tested in straight line: the halves are compared by packed 16-bit minima, and, because a
+// group fills its slots in order, it has room while its last half is zero and the first free word is
+// the first one whose upper half is.  An id whose home group is full, or that lost the slot to
+// another lane, takes the probe loop from the start.
+__device__ __forceinline__ int vis16_insert(uint32_t *vis, int gbits, int idbits, uint32_t id) {
+    uint32_t home, lo1;
+    vis16_key(id, idbits, gbits, home, lo1);
+    uint32_t *grp = vis + (home << 2);
+    const uint4 v = *reinterpret_cast<const uint4 *>(grp);
+    const uint32_t ee = lo1 * 0x00010001u;
+    const uint32_t t = pk_min16(pk_min16(v.x ^ ee, v.y ^ ee), pk_min16(v.z ^ ee, v.w ^ ee));
+    if ((t & 0xffffu) == 0u || t < 0x10000u) return 0;
+    int r = 2;
+    if (v.w < 0x10000u) {
+        const bool fx = v.x >= 0x10000u, fy = v.y >= 0x10000u, fz = v.z >= 0x10000u;
+        const uint32_t old = fz ? v.w : fy ? v.z : fx ? v.y : v.x;
+        const uint32_t wi = fz ? 3u : fy ? 2u : fx ? 1u : 0u;
+        const uint32_t nw = old == 0u ? lo1 : (old | (lo1 << 16));
+        r = atomicCAS(&grp[wi], old, nw) == old ? 1 : 2;
+        lds_fence();
+    }
+    if (r == 2) r = vis16_probe(vis, gbits, home, lo1);
+    return r;
 }
 __device__ __forceinline__ bool vis16_test(const uint32_t *vis, int gbits, int idbits, uint32_t id) {
     uint32_t home, lo1;
@@ -392,20 +434,46 @@ __device__ __forceinline__ float finish_f32(float s, float lena, float lenv) {
     return sign * (s * s / lena / lenv);
 }
 
-// One lane, sequential over the dimensions in the CPU's order (exact fallback).
+// One lane, sequential over the dimensions in the CPU's order (exact fallback).  Both operands are
+// read in 16-byte units; the row and the query are zero past dim, and a zero product leaves the sum
+// as it is.  The row's units are loaded SEQ_AHEAD at a time one block ahead of the additions, so the
+// chain of double additions does not wait for memory.
+constexpr int SEQ_AHEAD = 4;
 template <int METRIC>
 __device__ double seq_sum(const float *row, const float *qv, int dim) {
+    const float4 *r4 = reinterpret_cast<const float4 *>(row);
+    const float4 *q4 = reinterpret_cast<const float4 *>(qv);
+    const int nu = (dim + 3) >> 2;
+    float4 nx[SEQ_AHEAD];
+#pragma unroll
+    for (int t = 0; t < SEQ_AHEAD; ++t) nx[t] = r4[min(t, nu - 1)];
     double s = 0.0;
-    for (int i = 0; i < dim; ++i) {
-        float x = row[i], q = qv[i];
+    const auto add = [&](float x, float q) {
         float p;
         if (METRIC == M_L2) {
-            float d = x - q;
+            const float d = x - q;
             p = d * d;
         } else {
             p = x * q;
         }
         s += (double)p;
+    };
+    for (int j = 0; j < nu; j += SEQ_AHEAD) {
+        float4 x[SEQ_AHEAD];
+#pragma unroll
+        for (int t = 0; t < SEQ_AHEAD; ++t) x[t] = nx[t];
+#pragma unroll
+        for (int t = 0; t < SEQ_AHEAD; ++t) nx[t] = r4[min(j + SEQ_AHEAD + t, nu - 1)];
+#pragma unroll
+        for (int t = 0; t < SEQ_AHEAD; ++t) {
+            if (j + t < nu) {
+                const float4 q = q4[j + t];
+                add(x[t].x, q.x);
+                add(x[t].y, q.y);
+                add(x[t].z, q.z);
+                add(x[t].w, q.w);
+            }
+        }
     }
     return s;
 }
@@ -444,12 +512,59 @@ __device__ __forceinline__ void decode_unit(const uint4 u, float (&x)[Store<STOR
     }
 }
 
-// Distances of the m candidates cid[0..m): returns lane c's key (c < m).
-// SUB lanes share one row; each lane keeps its share of all rows of a pass in registers
-// (up to NVU 16-byte units) so every row load of the pass is issued before the first use.
+// sum over the SUB lanes that share a row: xor steps SUB/2 .. 1, the last four as DPP moves inside a
+// row of 16 lanes (a rotation by 4 stands for xor 4: after the xor 8 step lanes i and i ^ 8 agree)
+template <int CTRL> __device__ __forceinline__ float dpp_f(float x) {
+    return __uint_as_float(dpp32<CTRL>(__float_as_uint(x)));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_d(double x) {
+    return __longlong_as_double((long long)dpp64<CTRL>((uint64_t)__double_as_longlong(x)));
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_ROR4 = 0x124, DPP_ROR8 = 0x128;
+template <int SUB> __device__ __forceinline__ float sub_sum(float x) {
+    if constexpr (SUB > 16)
+        for (int o = SUB / 2; o > 8; o >>= 1) x += __shfl_xor(x, o);
+    if constexpr (SUB > 8) x += dpp_f<DPP_ROR8>(x);
+    if constexpr (SUB > 4) x += dpp_f<DPP_ROR4>(x);
+    x += dpp_f<DPP_XOR2>(x);
+    x += dpp_f<DPP_XOR1>(x);
+    return x;
+}
+template <int SUB> __device__ __forceinline__ double sub_sum(double x) {
+    if constexpr (SUB > 16)
+        for (int o = SUB / 2; o > 8; o >>= 1) x += __shfl_xor(x, o);
+    if constexpr (SUB > 8) x += dpp_d<DPP_ROR8>(x);
+    if constexpr (SUB > 4) x += dpp_d<DPP_ROR4>(x);
+    x += dpp_d<DPP_XOR2>(x);
+    x += dpp_d<DPP_XOR1>(x);
+    return x;
+}
+template <int SUB> __device__ __forceinline__ uint32_t sub_min(uint32_t x) {
+    if constexpr (SUB > 16)
+        for (int o = SUB / 2; o > 8; o >>= 1) x = min(x, (uint32_t)__shfl_xor((int)x, o));
+    if constexpr (SUB > 8) x = min(x, dpp32<DPP_ROR8>(x));
+    if constexpr (SUB > 4) x = min(x, dpp32<DPP_ROR4>(x));
+    x = min(x, dpp32<DPP_XOR2>(x));
+    x = min(x, dpp32<DPP_XOR1>(x));
+    return x;
+}
+
+// the candidate whose key eval_candidates leaves in this lane: pass p = lane % SUB, group lane / SUB
+template <int SUB> __device__ __forceinline__ int cand_of_lane() {
+    return (lane_id() % SUB) * (64 / SUB) + lane_id() / SUB;
+}
+
+// Distances of the m candidates cid[0..m): lane l returns the key of candidate cand_of_lane<SUB>()
+// (+inf when that is not below m).  SUB lanes share one row; each lane keeps its share of all rows of
+// a pass in registers (up to NVU 16-byte units) so every row load of the pass is issued before the
+// first use.  All SUB lanes of a row hold its sum, so the lane that keeps the key of pass p is
+// simply the row's lane p: no key moves between lanes.  The units of a pass are processed in straight
+// line (units past the row are clamped and their sum dropped by a select), so that the query's LDS
+// reads and the row loads are all in flight together; with a branch per unit each unit waited for
+// its own LDS reads.
 template <int METRIC, bool EXACT, int STORE, int SUB, int NVU, class Key>
-__device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, uint32_t cand, const uint32_t *cid,
-                                               const float *qv, float lenv) {
+__device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, const uint32_t *cid, const float *qv,
+                                               float lenv) {
     constexpr int EPU = Store<STORE>::EPU;
     const int lane = lane_id();
     constexpr int G = 64 / SUB;
@@ -459,43 +574,57 @@ __device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, uin
     bool redo = false;
     for (int base = 0; base < m; base += G) {
         const int c = base + g;
-        const bool valid = c < m;
-        const uint32_t id = valid ? cid[c] : 0u;
-        const uint4 *row = (STORE == ST_F32)
-                               ? reinterpret_cast<const uint4 *>(P.data + (size_t)id * (size_t)P.ld)
-                               : reinterpret_cast<const uint4 *>(P.data_lp + (size_t)id * P.lp_stride);
-        const float scale = (STORE != ST_F32 && valid) ? P.scale[id] : 1.0f;
-        float facc = 0.0f;
-        double dacc = 0.0, sab = 0.0;
-        int mn = 0x3fffffff;
-        for (int j0 = 0; j0 < nu; j0 += NVU * SUB) {
-            uint4 u[NVU];
-            if (valid) {
-                // indices past the row are clamped (and skipped below): one predicate for all loads
+        if (c < m) {
+            const uint32_t id = cid[c];
+            const uint4 *row = (STORE == ST_F32)
+                                   ? reinterpret_cast<const uint4 *>(P.data + (size_t)id * (size_t)P.ld)
+                                   : reinterpret_cast<const uint4 *>(P.data_lp + (size_t)id * P.lp_stride);
+            const float scale = (STORE != ST_F32) ? P.scale[id] : 1.0f;
+            const float lena = (METRIC == M_COS) ? P.norms[id] : 0.0f;
+            float facc = 0.0f;
+            double dacc = 0.0, sab = 0.0;
+            uint32_t umin = ~0u;
+            // NVC units per lane from unit j0 on; MASKED: some may lie past the row
+            const auto block = [&](int j0, auto masked, auto units) {
+                constexpr bool MASKED = decltype(masked)::value;
+                constexpr int NVC = decltype(units)::value;
+                uint4 u[NVC];
 #pragma unroll
-                for (int v = 0; v < NVU; ++v) u[v] = row[min(j0 + sl + v * SUB, nu - 1)];
-            }
+                for (int v = 0; v < NVC; ++v) {
+                    const int j = j0 + sl + v * SUB;
+                    u[v] = row[MASKED ? min(j, nu - 1) : j];
+                }
 #pragma unroll
-            for (int v = 0; v < NVU; ++v) {
-                const int j = j0 + sl + v * SUB;
-                if (valid && j < nu) {
-                    float x[EPU];
+                for (int v = 0; v < NVC; ++v) {
+                    const int j = j0 + sl + v * SUB;
+                    const int jq = MASKED ? min(j, nu - 1) : j;
+                    float x[EPU], q[EPU];
                     decode_unit<STORE>(u[v], x);
-                    const float *q = qv + j * EPU;
+#pragma unroll
+                    for (int t = 0; t < EPU; t += 4) {
+                        const float4 q4 = *reinterpret_cast<const float4 *>(qv + jq * EPU + t);
+                        q[t] = q4.x; q[t + 1] = q4.y; q[t + 2] = q4.z; q[t + 3] = q4.w;
+                    }
+                    const bool in = !MASKED || j < nu;
                     if constexpr (!EXACT) {
+                        float f = facc;
 #pragma unroll
                         for (int t = 0; t < EPU; ++t) {
                             const float xv = (STORE == ST_F32) ? x[t] : x[t] * scale;
                             if (METRIC == M_L2) {
                                 const float d = xv - q[t];
-                                facc += d * d;
+                                f += d * d;
                             } else {
-                                facc += xv * q[t];
+                                f += xv * q[t];
                             }
                         }
+                        facc = in ? f : facc;
                     } else {
-                        // float products (rounded), double accumulation; exact in any order when
-                        // all products are multiples of 2^mn and sum |p| < 2^(mn+53)
+                        // float products (rounded), double accumulation; exact in any order when all
+                        // products are multiples of 2^mn and sum |p| < 2^(mn+53).  2^mn from the
+                        // smallest nonzero product's exponent (its last mantissa bit)
+                        double f = dacc, sf = sab;
+                        uint32_t um = umin;
 #pragma unroll
                         for (int t = 0; t < EPU; ++t) {
                             float pr;
@@ -505,54 +634,54 @@ __device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, uin
                             } else {
                                 pr = x[t] * q[t];
                             }
-                            dacc += (double)pr;
-                            sab += (double)fabsf(pr);
-                            mn = min(mn, lsb_exp(pr));
+                            f += (double)pr;
+                            if (METRIC != M_L2) sf += (double)fabsf(pr);
+                            um = min(um, (__float_as_uint(pr) & 0x7fffffffu) - 1u);
                         }
+                        dacc = in ? f : dacc;
+                        sab = in ? sf : sab;
+                        umin = in ? um : umin;
                     }
                 }
+            };
+            using T_ = std::true_type;
+            using F_ = std::false_type;
+            constexpr int CH = NVU * SUB;
+            if (NVU == 2 && nu <= SUB) {
+                block(0, T_{}, std::integral_constant<int, 1>{});
+            } else {
+                int j0 = 0;
+                for (; j0 + CH <= nu; j0 += CH) block(j0, F_{}, std::integral_constant<int, NVU>{});
+                if (j0 < nu) block(j0, T_{}, std::integral_constant<int, NVU>{});
             }
-        }
-        Key k;
-        bool seq = false;
-        if constexpr (!EXACT) {
-#pragma unroll
-            for (int o = SUB / 2; o > 0; o >>= 1) facc += __shfl_xor(facc, o);
-            const float lena = (METRIC == M_COS && valid) ? P.norms[id] : 0.0f;
-            k = Key::make_f(finish_f32<METRIC>(facc, lena, lenv), id);
-        } else {
-#pragma unroll
-            for (int o = SUB / 2; o > 0; o >>= 1) {
-                dacc += __shfl_xor(dacc, o);
-                sab += __shfl_xor(sab, o);
-                mn = min(mn, __shfl_xor(mn, o));
+            Key k;
+            bool seq = false;
+            if constexpr (!EXACT) {
+                k = Key::make_f(finish_f32<METRIC>(sub_sum<SUB>(facc), lena, lenv), id);
+            } else {
+                dacc = sub_sum<SUB>(dacc);
+                const double tot = METRIC == M_L2 ? dacc : sub_sum<SUB>(sab);
+                umin = sub_min<SUB>(umin);
+                // every product zero (umin still all ones), or tot < 2^(mn + 53) with one bit to spare for
+                // the rounding of tot itself: biased exponent of tot below mn + 53 + 1023 - 1
+                const int mn = max((int)(umin >> 23), 1) - 150;
+                const int te = (int)(((uint64_t)__double_as_longlong(tot) >> 52) & 2047u);
+                seq = umin != ~0u && te - 1023 > mn + 51;
+                k = Key::make_d(finish_exact<METRIC>(dacc, lena, lenv), id);
             }
-            seq = !((sab == 0.0) || (mn < 0x3fffffff && sab < ldexp(1.0, mn + 53)));
-            const float lena = (METRIC == M_COS && valid) ? P.norms[id] : 0.0f;
-            k = Key::make_d(finish_exact<METRIC>(dacc, lena, lenv), id);
-        }
-        // lane c (base <= c < base + G) takes the key of group c - base
-        const int src = ((lane - base) & (G - 1)) * SUB;
-        Key got;
-        if constexpr (!EXACT) {
-            got.v = ((uint64_t)(uint32_t)__shfl((int)(k.v >> 32), src) << 32) | (uint32_t)__shfl((int)k.v, src);
-        } else {
-            got.d = ((uint64_t)(uint32_t)__shfl((int)(k.d >> 32), src) << 32) | (uint32_t)__shfl((int)k.d, src);
-            got.i = (uint32_t)__shfl((int)k.i, src);
-            got.pad = 0u;
-        }
-        const bool seq_got = __shfl((int)seq, src) != 0;
-        if (lane >= base && lane < base + G && lane < m) {
-            mine = got;
-            redo = seq_got;
+            if (base == sl * G) {
+                mine = k;
+                redo = seq;
+            }
         }
     }
     if constexpr (EXACT) {
         // sequential re-evaluation in the CPU's order, one lane per flagged candidate
         if (redo) {
-            const double s = seq_sum<METRIC>(P.data + (size_t)cand * (size_t)P.ld, qv, P.dim);
-            const float lena = (METRIC == M_COS) ? P.norms[cand] : 0.0f;
-            mine = Key::make_d(finish_exact<METRIC>(s, lena, lenv), cand);
+            const uint32_t id = mine.id();
+            const float lena = (METRIC == M_COS) ? P.norms[id] : 0.0f;
+            const double s = seq_sum<METRIC>(P.data + (size_t)id * (size_t)P.ld, qv, P.dim);
+            mine = Key::make_d(finish_exact<METRIC>(s, lena, lenv), id);
         }
     }
     return mine;
@@ -574,7 +703,7 @@ __device__ __forceinline__ KeyF wave_min(KeyF k) {
 // 64 equal chunks (one LDS read per lane) and keeps the chunk holding the boundary.
 template <class Key, class Pred>
 __device__ __forceinline__ int prefix_count(const Key *arr, int n, Pred below) {
-    const int lane = lane_id();
+    const int lane = rare_lane();
     int lo = 0, len = n;
     while (len > 64) {
         const int stride = (len + 63) >> 6;
@@ -594,7 +723,7 @@ __device__ __forceinline__ int prefix_count(const Key *arr, int n, Pred below) {
 // arr[p, e) moves to arr[p + 1, e + 1) and arr[p] = x (blocks of 64, last block first, so each
 // block is read before the block below it writes into its first slot)
 template <class Key> __device__ __forceinline__ void shift_insert(Key *arr, int p, int e, const Key &x) {
-    const int lane = lane_id();
+    const int lane = rare_lane();
     for (int blk = (e - 1) >> 6; blk >= (p >> 6) && e > p; --blk) {
         const int i = blk * 64 + lane;
         const bool live = i >= p && i < e;
@@ -620,7 +749,7 @@ template <class Key> __device__ __forceinline__ Key kmax(const Key &a, const Key
 // sequence ascends where (lane & K) == 0 and descends otherwise (K = 64: ascending).
 template <class Key>
 __device__ __forceinline__ Key bitonic_steps(Key v, int K, int J) {
-    const int lane = lane_id();
+    const int lane = rare_lane();
     const bool up = (lane & K) == 0;
     for (int j = J >> 1; j > 0; j >>= 1) {
         const Key o = shfl_key(v, lane ^ j);
@@ -639,7 +768,7 @@ __device__ __forceinline__ Key bitonic_steps(Key v, int K, int J) {
 constexpr int SEL_INSERT = 16;
 template <class Key>
 __device__ __forceinline__ Key select64(const Key *arr, int n) {
-    const int lane = lane_id();
+    const int lane = rare_lane();
     Key best = (lane < n) ? arr[lane] : Key::inf();
     // two blocks' loads are in flight while one is sorted or scanned (two register slots, the
     // loop unrolled by two, so no slot is copied while its load is in flight)
@@ -678,7 +807,7 @@ __device__ __forceinline__ Key select64(const Key *arr, int n) {
 // from the top; hist: 256 u32 of this wave's LDS.
 template <class Key>
 __device__ uint64_t select_dk(const Key *arr, int n, int r, uint32_t *hist) {
-    const int lane = lane_id();
+    const int lane = rare_lane();
     uint64_t prefix = 0, pmask = 0;
     uint32_t need = (uint32_t)r;
     for (int shift = Key::DKBITS - 8; shift >= 0; shift -= 8) {
@@ -731,7 +860,7 @@ __device__ uint64_t select_dk(const Key *arr, int n, int r, uint32_t *hist) {
 // the loop unrolled by two), and block j's own slots are written only after its load is used.
 template <class Key, class Keep>
 __device__ __forceinline__ int compact(Key *arr, int n, Keep keep_fn) {
-    const int lane = lane_id();
+    const int lane = rare_lane();
     int out = 0;
     Key na = (lane < n) ? arr[lane] : Key::inf();
     Key nb = (64 + lane < n) ? arr[64 + lane] : Key::inf();
@@ -799,6 +928,13 @@ __device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin
 
 // ---------------------------------------------------------------- the search kernel
 
+// What bounds it: the chain of one expansion (pop, visited probe, row gather, queue insert), most of
+// it instruction and LDS latency, so its work is kept straight: probes and distances without
+// branches per slot or unit, sums by DPP moves, keys inserted by lane shifts, no key moved between
+// lanes through LDS.  Against the chain with LDS scatters, shuffles and per-unit branches (1M x 128
+// L2 unless said; one launch): 10,000 queries at pq 704 13.75 -> 12.57 ms, 3,001 at pq 200 2.06 ->
+// 1.79 ms, 48 at pq 128 816 -> 666 us; 5,000 cosine queries of 16 dimensions in exact arithmetic
+// 1,005 -> 752 us; 1,000 queries on FP8 rows of 960 dimensions 2.16 -> 1.62 ms.
 // One query on one wave: qi is the query, slot_q the wave's spill table, smem its LDS.
 // BAGL: the queue's bag sits in the wave's LDS slice after the query (qcap keys) instead of in
 // global memory -- for latency-bound launches with few waves per CU, where a refill or a
@@ -825,12 +961,11 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     const bool bloom = P.bloom_k > 0;
     const uint32_t vis_bytes = bloom ? (4u << P.hlog) : H * (P.vis16 ? 2u : 4u);
     const int gbits = P.hlog - 3;                               // compact table: groups of 8
-    Key *S = reinterpret_cast<Key *>(smem + vis_bytes);        // merge scratch, QH keys
-    // the best list's front: LDS after the scratch, or (bglob: float32 rows, global bag) the
+    // the best list's front: LDS after the visited table, or (bglob: float32 rows, global bag) the
     // slot's global region after its bag
     static_assert(!BG || (STORE == ST_F32 && !BAGL), "the global front needs float32 rows and a global bag");
     constexpr bool bglob = BG;
-    Key *B = S + QH;
+    Key *B = reinterpret_cast<Key *>(smem + vis_bytes);
     // the front (computed where used, in rare paths, so that no registers hold a global
     // pointer through the loop)
     const auto Bf = [&]() -> Key * {
@@ -925,6 +1060,37 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     int tb = 0;
     // the queue head lives in registers: lanes [h, h + nq) hold its keys in ascending order
     Key hq = Key::inf();
+    int bn = 0;          // bag entries: unsorted, all above T
+    Key T = Key::inf();  // head entries <= T < bag entries (+inf while the bag is empty)
+
+    // A wave-uniform key into the register head: a shift of the lanes below its rank into the consumed
+    // lanes in front of the head, or, with none, of the lanes above it; then a full head gives its
+    // largest key to the bag and lowers T.  Keys are distinct.  One key costs a compare, two lane
+    // shifts and four selects and no LDS access; a merge that scattered head and new keys through LDS
+    // took two dependent LDS round trips per expansion and the same work per new key.
+    const auto push_head = [&](const Key &o) {
+        const uint64_t below = ballot(lt(hq, o)) & (low_bits(nq) << h);
+        const int r = __popcll(below);
+        if (h > 0) {
+            hq = ksel(in_mask(below >> 1), shl1(hq), hq);
+            hq = ksel(in_mask(1ull << (h - 1 + r)), o, hq);
+            --h;
+            ++nq;
+        } else {
+            const bool full = nq == QH;
+            if (full) {
+                const Key top = hq.rl(QH - 1);
+                if (lane == 0) Bg[bn] = ksel(r == QH, o, top);
+                ++bn;
+            }
+            if (r < QH) {
+                hq = ksel(in_mask(low_bits(r)), hq, shr1(hq));
+                hq = ksel(in_mask(1ull << r), o, hq);
+            }
+            if (full) T = hq.rl(QH - 1);
+            else ++nq;
+        }
+    };
 
     // start vertices (graph.h:175-181: vertex 0; the learned form passes its own), each
     // entered once through the visited set and placed in the queue in (dist, id) order
@@ -950,14 +1116,8 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         if (fresh) cid[lanes_below(fm)] = sid;
         nvis = (uint32_t)m0;
         lds_fence();
-        const uint32_t cand0 = (lane < m0) ? cid[lane] : 0u;
-        const Key k0 = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m0, cand0, cid, qv, lenv);
-        int rank = 0;
-        for (int j = 0; j < m0; ++j) rank += lt(k0.rl(j), k0) ? 1 : 0;
-        if (lane < m0) S[rank] = k0;
-        lds_fence();
-        hq = (lane < m0) ? S[lane] : Key::inf();
-        nq = m0;
+        const Key k0 = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m0, cid, qv, lenv);
+        for (uint64_t bits = ballot(cand_of_lane<SUB>() < m0); bits; bits &= bits - 1) push_head(k0.rl(__builtin_ctzll(bits)));
         lds_fence();
     }
     const int max_steps = P.steps_arr ? min(P.steps_arr[qi], P.max_steps) : P.max_steps;
@@ -976,8 +1136,6 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         return P.graph[(size_t)v * (size_t)P.gstride + (uint32_t)min(lane, P.gstride - 1)];
     };
 
-    int bn = 0;          // bag entries: unsorted, all above T
-    Key T = Key::inf();  // head entries <= T < bag entries (+inf while the bag is empty)
     // one expansion; returns true to leave the loop
     const auto expand = [&](auto parity) -> bool {
         constexpr int X = decltype(parity)::value, Y = 1 - X;
@@ -1029,39 +1187,43 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         // Expansions come out in nearly ascending order, so `now` almost always lands in the
         // register tail: one compare and a lane shift, no LDS round trip.
         {
+            // the tail's entries below `now` are its first c lanes, so the ballot itself is the mask of the
+            // lanes that keep their entry
             const uint64_t below = ballot(lt(bt, now));
-            const bool in_tail = tb == 0 || (below & 1ull);
-            const int p = in_tail ? tb + __popcll(below)
-                                  : (front_fence(), prefix_count(Bf(), tb, [&](const Key &e) { return lt(e, now); }));
+            int p = tb + __popcll(below);
+            if (tb > 0 && !(below & 1ull)) {  // below the tail: in the front, or right at the tail's start
+                front_fence();
+                p = prefix_count(Bf(), tb, [&](const Key &e) { return lt(e, now); });
+            }
             if (p < k && lane == 0) settle = steps;
             if (p < pq) {
-                const int j = p - tb;  // tail lane of the new entry; negative: it lands in the front
-                if (nbest >= 64 && nbest < pq) {
-                    // growing past 64 entries: tb advances by one and position tb joins the front
-                    if (j >= 0) {
-                        // the 65 entries [tb, nbest] with `now` at j: the first goes to the front,
-                        // lanes below j - 1 take their upper neighbour's entry
-                        if (lane == 0) Bf()[tb] = ksel(j == 0, now, bt);
-                        const Key up = shl1(bt);
-                        bt = ksel(lane < j - 1, up, ksel(lane == j - 1, now, bt));
+                if (p >= tb) {
+                    const int c = p - tb;
+                    if (nbest >= 64 && nbest < pq) {
+                        // growing past 64 entries: the smallest of the 65 entries [tb, nbest] with `now`
+                        // at c goes to the front, lanes below c - 1 take their upper neighbour's entry
+                        if (lane == 0) Bf()[tb] = ksel(c == 0, now, bt);
+                        bt = ksel(in_mask(below >> 1), shl1(bt), bt);
+                        if (c > 0) bt = ksel(in_mask(1ull << (c - 1)), now, bt);
+                        ++tb;
                     } else {
-                        // front [p, tb) moves to [p + 1, tb + 1); the tail keeps its entries
-                        shift_insert(Bf(), p, tb, now);  // (a front in global memory: after the fence above)
+                        // below 64 entries (tb = 0), or full (the entry at pq - 1 leaves)
+                        bt = ksel(in_mask(below), bt, shr1(bt));
+                        bt = ksel(in_mask(1ull << c), now, bt);
+                        if (nbest == pq && pq < 64) bt = ksel(in_mask(1ull << pq), Key::inf(), bt);
                     }
+                } else if (nbest < pq) {
+                    // front [p, tb) moves to [p + 1, tb + 1); the tail keeps its entries
+                    shift_insert(Bf(), p, tb, now);  // (a front in global memory: after the fence above)
                     ++tb;
-                } else if (j >= 0) {
-                    // below 64 entries (tb = 0), or full (the entry at pq - 1 leaves)
-                    const Key dn = shr1(bt);
-                    bt = ksel(lane < j, bt, ksel(lane == j, now, dn));
                 } else {
-                    // full, `now` in the front: the front's last entry moves into the tail
+                    // full: the front's last entry moves into the tail, the entry at pq - 1 leaves
                     const Key fl = Bf()[tb - 1];
                     shift_insert(Bf(), p, tb - 1, now);
                     const Key dn = shr1(bt);
                     bt = ksel(lane == 0, fl, dn);
                 }
                 nbest = min(nbest + 1, pq);
-                bt = ksel(lane >= nbest - tb, Key::inf(), bt);
                 if (nbest == pq) bmax = bt.rl(pq - 1 - tb).dk();
                 lds_fence();
             }
@@ -1125,28 +1287,30 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         }
         if (m == 0) return false;
         lds_fence();
-        const uint32_t cand = (lane < m) ? cid[lane] : 0u;
         Key mine;
+        bool have = cand_of_lane<SUB>() < m;
         bool cached = false;
         if constexpr (HELP) {
             if (use_cache) {
                 // every candidate's distance in the helper's cache: no gather
-                const uint64_t ce = (lane < m) ? dcache[duo_slot(cand)] : ~0ull;
-                const bool hit = lane < m && (uint32_t)ce == cand;
-                if (ballot(lane < m && !hit) == 0ull) {
-                    mine = KeyF{(lane < m) ? ce : ~0ull};
+                const uint64_t ce = fresh ? dcache[duo_slot(r)] : ~0ull;
+                const bool hit = fresh && (uint32_t)ce == r;
+                if (ballot(fresh && !hit) == 0ull) {
+                    mine = KeyF{ce};
+                    have = fresh;
                     cached = true;
                     cache_hits += l0;
                 }
             }
         }
-        if (!cached) mine = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m, cand, cid, qv, lenv);
+        if (!cached) mine = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m, cid, qv, lenv);
 
         // ---- the candidates: at most T into the sorted head, above T into the bag
         const uint64_t cut = (nbest == pq) ? bmax : ~0ull;  // drop distance keys above cut
-        const bool surv = lane < m && mine.dk() <= cut;
+        const bool surv = have && mine.dk() <= cut;
         if (ballot(surv) == 0ull) return false;
-        if (bn + 62 > P.qcap) {
+        // (a row has at most 63 neighbours, each of which adds at most one key to the bag)
+        if (bn + 63 > P.qcap) {
             // make room: drop bag entries beyond the pq-th smallest distance of head + bag
             // (ties kept) or beyond bmax; none of them can be expanded before the stop rule
             uint64_t dcut = (nbest == pq) ? bmax : ~0ull;
@@ -1157,7 +1321,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
             bn = keep_dk_upto(Bg, bn, dcut);
             if constexpr (!BAGL) vm_drain();
             if (bn == 0) T = Key::inf();
-            if (bn + 62 > P.qcap) {  // the tie group at the pq-th distance exceeds the slack
+            if (bn + 63 > P.qcap) {  // the tie group at the pq-th distance exceeds the slack
                 flags |= F_Q_OVF;
                 return true;
             }
@@ -1167,44 +1331,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         const uint64_t bm = ballot(to_b);
         if (to_b) Bg[bn + lanes_below(bm)] = mine;
         bn += __popcll(bm);
-        const uint64_t sm = ballot(to_q);
-        const int ms = __popcll(sm);
-        if (ms > 0) {
-            // merge into the register head.  A head key moves down by the h consumed lanes and
-            // up by the survivors below it; a survivor lands after the head keys and survivors
-            // below it.  Keys are distinct, so the destinations are a permutation of
-            // [0, nq + ms); those past the last lane go to the bag (they exceed every key that
-            // stays), the rest pass through the LDS scratch.
-            const bool live = lane >= h && lane < h + nq;
-            int cnt = 0, sdst = 0;
-            for (uint64_t bits = sm; bits; bits &= bits - 1) {
-                const int j = __builtin_ctzll(bits);
-                const Key o = mine.rl(j);
-                cnt += (live && lt(o, hq)) ? 1 : 0;
-                const int d = __popcll(ballot(live && lt(hq, o))) + __popcll(ballot(to_q && lt(mine, o)));
-                if (lane == j) sdst = d;
-            }
-            const int hdst = lane - h + cnt;
-            const int nn = nq + ms;
-            if (nn > QH) {
-                if (live && hdst >= QH) Bg[bn + hdst - QH] = hq;
-                if (to_q && sdst >= QH) Bg[bn + sdst - QH] = mine;
-            }
-            if (live && hdst < QH) S[hdst] = hq;
-            if (to_q && sdst < QH) S[sdst] = mine;
-            lds_fence();
-            hq = (lane < nn) ? S[lane] : Key::inf();
-            h = 0;
-            if (nn > QH) {
-                // the head keeps its QH smallest; T drops to its new largest key
-                bn += nn - QH;
-                nq = QH;
-                T = hq.rl(QH - 1);
-            } else {
-                nq = nn;
-            }
-            lds_fence();
-        }
+        for (uint64_t bits = ballot(to_q); bits; bits &= bits - 1) push_head(mine.rl(__builtin_ctzll(bits)));
         // the queue head may have changed: refresh the prefetch target only if it did
         if (nq > 0 && hq.rl(h).id() != pid[Y]) {
             pid[Y] = hq.rl(h).id();
@@ -1233,9 +1360,8 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
                 const int c = min(64, nbest - base);
                 if (lane < c) cid[lane] = B[base + lane].id();
                 lds_fence();
-                const uint32_t cand = (lane < c) ? cid[lane] : 0u;
-                const Key ex = eval_candidates<METRIC, false, ST_F32, 4, 8, Key>(P, c, cand, cid, qv, lenv);
-                if (lane < c) B[base + lane] = ex;
+                const Key ex = eval_candidates<METRIC, false, ST_F32, 4, 8, Key>(P, c, cid, qv, lenv);
+                if (cand_of_lane<4>() < c) B[base + cand_of_lane<4>()] = ex;
                 lds_fence();
             }
             for (int r = 0; r < k; ++r) {
@@ -1327,12 +1453,12 @@ __device__ void duo_helper(const SearchParams &P, unsigned char *slice, unsigned
     DuoMail *mail = reinterpret_cast<DuoMail *>(duo);
     uint64_t *dcache = reinterpret_cast<uint64_t *>(duo + sizeof(DuoMail));
     uint32_t *hid = reinterpret_cast<uint32_t *>(dcache + DUO_CACHE);
-    // the search wave's layout (search_query): visited | 64 keys | pq keys (not with bglob) | 256 u32 | qv
+    // the search wave's layout (search_query): visited | pq keys (not with bglob) | 256 u32 | qv
     const uint32_t H = 1u << P.hlog;
     const uint32_t vis_bytes = H * (P.vis16 ? 2u : 4u);
     const uint32_t *vis = reinterpret_cast<const uint32_t *>(slice);
-    const KeyF *S = reinterpret_cast<const KeyF *>(slice + vis_bytes);
-    const uint32_t *cid = reinterpret_cast<const uint32_t *>(S + 64 + (BG ? 0 : ((P.pq + 1) & ~1)));
+    const KeyF *B = reinterpret_cast<const KeyF *>(slice + vis_bytes);
+    const uint32_t *cid = reinterpret_cast<const uint32_t *>(B + (BG ? 0 : ((P.pq + 1) & ~1)));
     const float *qv = reinterpret_cast<const float *>(cid + 256);
     uint32_t my_epoch = 0u, last_t = 0u;
     float lenv = 0.0f;
@@ -1365,9 +1491,8 @@ __device__ void duo_helper(const SearchParams &P, unsigned char *slice, unsigned
         if (m == 0) continue;
         if (want) hid[lanes_below(fm)] = r;
         lds_fence();
-        const uint32_t cand = (lane < m) ? hid[lane] : 0u;
-        const KeyF k = eval_candidates<METRIC, false, STORE, SUB, NV, KeyF>(P, m, cand, hid, qv, lenv);
-        if (lane < m) dcache[duo_slot(cand)] = k.v;
+        const KeyF k = eval_candidates<METRIC, false, STORE, SUB, NV, KeyF>(P, m, hid, qv, lenv);
+        if (cand_of_lane<SUB>() < m) dcache[duo_slot(k.id())] = k.v;
         lds_fence();
     }
 }

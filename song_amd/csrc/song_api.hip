@@ -310,13 +310,13 @@ extern "C" int song_index_integer_valued(const song_index *ix) { return ix ? ix-
 // ---------------------------------------------------------------- launch planning
 
 // must match the per-wave layout of search_query: visited (2^hlog slots of 4 or, compact, 2
-// bytes) | head merge scratch (64 keys) | best (pq rounded to even; not with bglob) | 256
+// bytes) | best (pq rounded to even; not with bglob) | 256
 // candidate ids / radix bins | query (the head is in registers, the bag in global memory)
 size_t song::lds_bytes(bool exact, int pq, int qcap, int hlog, int qld, int vis16, int bloom_k, int bag_lds,
                        int bglob) {
     size_t key = exact ? 16 : 8;
     const size_t vis = bloom_k > 0 ? ((size_t)4 << hlog) : ((size_t)(vis16 ? 2 : 4) << hlog);
-    return vis + (size_t)64 * key + (bglob ? 0 : (size_t)((pq + 1) & ~1) * key) + 256 * 4 + (size_t)qld * 4 +
+    return vis + (bglob ? 0 : (size_t)((pq + 1) & ~1) * key) + 256 * 4 + (size_t)qld * 4 +
            (bag_lds ? (size_t)qcap * key : 0);
 }
 
