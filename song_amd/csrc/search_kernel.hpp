@@ -436,44 +436,57 @@ __device__ __forceinline__ float finish_f32(float s, float lena, float lenv) {
 
 // One lane, sequential over the dimensions in the CPU's order (exact fallback).  Both operands are
 // read in 16-byte units; the row and the query are zero past dim, and a zero product leaves the sum
-// as it is.  The row's units are loaded SEQ_AHEAD at a time one block ahead of the additions, so the
-// chain of double additions does not wait for memory.
-constexpr int SEQ_AHEAD = 4;
-template <int METRIC>
+// as it is.  What bounds it is the chain of double additions, so everything else is kept off it: row
+// units are loaded in two alternating blocks of AHEAD, one in flight while the other is used, and a
+// block's query reads and products come before its additions.  Wide rows take 8 units a block;
+// narrow ones, whose sums are short and seldom need this, 1, which keeps the registers (and so the
+// waves per SIMD) of their kernels.  1,000 queries on 960 dimensions: 10.36 -> 9.47 ms; with 8 units for
+// rows of 16 dimensions too, 5,000 cosine queries took 988 instead of 752 us (two waves per SIMD).
+template <int METRIC, int AHEAD = 1>
 __device__ double seq_sum(const float *row, const float *qv, int dim) {
     const float4 *r4 = reinterpret_cast<const float4 *>(row);
     const float4 *q4 = reinterpret_cast<const float4 *>(qv);
     const int nu = (dim + 3) >> 2;
-    float4 nx[SEQ_AHEAD];
-#pragma unroll
-    for (int t = 0; t < SEQ_AHEAD; ++t) nx[t] = r4[min(t, nu - 1)];
     double s = 0.0;
-    const auto add = [&](float x, float q) {
-        float p;
+    const auto prod = [](float x, float q) {
         if (METRIC == M_L2) {
             const float d = x - q;
-            p = d * d;
-        } else {
-            p = x * q;
+            return d * d;
         }
-        s += (double)p;
+        return x * q;
     };
-    for (int j = 0; j < nu; j += SEQ_AHEAD) {
-        float4 x[SEQ_AHEAD];
+    float4 xa[AHEAD], xb[AHEAD];
+    const auto load = [&](float4 (&x)[AHEAD], int j) {
 #pragma unroll
-        for (int t = 0; t < SEQ_AHEAD; ++t) x[t] = nx[t];
+        for (int t = 0; t < AHEAD; ++t) x[t] = r4[min(j + t, nu - 1)];
+    };
+    const auto take = [&](float4 (&x)[AHEAD], int j) {
+        float4 q[AHEAD];
 #pragma unroll
-        for (int t = 0; t < SEQ_AHEAD; ++t) nx[t] = r4[min(j + SEQ_AHEAD + t, nu - 1)];
+        for (int t = 0; t < AHEAD; ++t) q[t] = q4[min(j + t, nu - 1)];
 #pragma unroll
-        for (int t = 0; t < SEQ_AHEAD; ++t) {
-            if (j + t < nu) {
-                const float4 q = q4[j + t];
-                add(x[t].x, q.x);
-                add(x[t].y, q.y);
-                add(x[t].z, q.z);
-                add(x[t].w, q.w);
-            }
+        for (int t = 0; t < AHEAD; ++t) {
+            // a unit past the row contributes zeros
+            const bool in = j + t < nu;
+            x[t].x = in ? prod(x[t].x, q[t].x) : 0.0f;
+            x[t].y = in ? prod(x[t].y, q[t].y) : 0.0f;
+            x[t].z = in ? prod(x[t].z, q[t].z) : 0.0f;
+            x[t].w = in ? prod(x[t].w, q[t].w) : 0.0f;
         }
+#pragma unroll
+        for (int t = 0; t < AHEAD; ++t) {
+            s += (double)x[t].x;
+            s += (double)x[t].y;
+            s += (double)x[t].z;
+            s += (double)x[t].w;
+        }
+    };
+    load(xa, 0);
+    for (int j = 0; j < nu; j += 2 * AHEAD) {
+        load(xb, j + AHEAD);
+        take(xa, j);
+        load(xa, j + 2 * AHEAD);
+        take(xb, j + AHEAD);
     }
     return s;
 }
@@ -680,7 +693,7 @@ __device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, con
         if (redo) {
             const uint32_t id = mine.id();
             const float lena = (METRIC == M_COS) ? P.norms[id] : 0.0f;
-            const double s = seq_sum<METRIC>(P.data + (size_t)id * (size_t)P.ld, qv, P.dim);
+            const double s = seq_sum<METRIC, (SUB >= 16 ? 8 : 1)>(P.data + (size_t)id * (size_t)P.ld, qv, P.dim);
             mine = Key::make_d(finish_exact<METRIC>(s, lena, lenv), id);
         }
     }

@@ -240,10 +240,18 @@ extern "C" int song_index_create(const float *data, uint64_t n, int dim, const u
 
     size_t dbytes = (size_t)n * ix->ld * sizeof(float);
     if (hipMalloc(&ix->d_data, dbytes) != hipSuccess) return cleanup(fail(SONG_E_HIP, "hipMalloc data %zu", dbytes));
-    if (hipMemset(ix->d_data, 0, dbytes) != hipSuccess) return cleanup(fail(SONG_E_HIP, "hipMemset data"));
-    if (hipMemcpy2D(ix->d_data, ix->ld * sizeof(float), data, dim * sizeof(float), dim * sizeof(float), n,
-                    hipMemcpyHostToDevice) != hipSuccess)
-        return cleanup(fail(SONG_E_HIP, "upload data"));
+    // rows of a multiple of four floats go up as they lie; others are padded with zeros, cleared
+    // before the copy starts
+    if (ix->ld == dim) {
+        if (hipMemcpy(ix->d_data, data, dbytes, hipMemcpyHostToDevice) != hipSuccess)
+            return cleanup(fail(SONG_E_HIP, "upload data"));
+    } else {
+        if (hipMemset(ix->d_data, 0, dbytes) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
+            return cleanup(fail(SONG_E_HIP, "hipMemset data"));
+        if (hipMemcpy2D(ix->d_data, ix->ld * sizeof(float), data, dim * sizeof(float), dim * sizeof(float), n,
+                        hipMemcpyHostToDevice) != hipSuccess)
+            return cleanup(fail(SONG_E_HIP, "upload data"));
+    }
     size_t gbytes = g32.size() * sizeof(uint32_t);
     if (hipMalloc(&ix->d_graph, gbytes) != hipSuccess) return cleanup(fail(SONG_E_HIP, "hipMalloc graph"));
     if (hipMemcpy(ix->d_graph, g32.data(), gbytes, hipMemcpyHostToDevice) != hipSuccess)
