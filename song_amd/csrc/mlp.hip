@@ -56,21 +56,16 @@ struct GemmArgs {
     long long sam, sak;
     const uint16_t *B;
     long long sbk, sbn;
-    float *C;  // float32 output or null
+    float *C;
     int ldc;
-    uint16_t *Cb;  // bf16 output or null
-    int ldcb;
-    const float *bias;      // per column, or null
-    const uint16_t *mask;   // zero the output where mask[m][n] <= 0 (ReLU backward), or null
-    int ldm;
-    int relu;
     float alpha;
 };
 
 constexpr int GBM = 64, GBN = 64, GBK = 16;
 
-// C[m][n] = alpha * sum_k A(m,k) B(k,n) (+ bias[n]) (ReLU) (mask), A(m,k) = A[m*sam + k*sak],
-// B(k,n) = B[k*sbk + n*sbn].  256 threads: 2x2 waves of 32x32, each 2x2 MFMA tiles.
+// C[m][n] = alpha * sum_k A(m,k) B(k,n), A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn], any
+// strides (song_gemm_bf16; the network's own products are tile_kernel's).  256 threads: 2x2 waves of
+// 32x32, each 2x2 MFMA tiles.
 __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
     __shared__ uint16_t As[GBM][GBK + 4];
     __shared__ uint16_t Bs[GBN][GBK + 4];
@@ -114,72 +109,274 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
             for (int j = 0; j < 4; ++j) {
                 const int m = m0 + wm + mi * 16 + 4 * (lane >> 4) + j;
                 const int n = n0 + wn + ni * 16 + (lane & 15);
+                if (m < g.M && n < g.N) g.C[(long long)m * g.ldc + n] = g.alpha * acc[mi][ni][j];
+            }
+}
+
+// ---------------------------------------------------------------- the network's products
+
+// The training products: operands whose rows are 16-byte aligned along one of their two directions.
+// A block computes BM x BN with 2 x 2 waves, BK of the contraction at a time, through two LDS buffers
+// of k-contiguous rows; the next PF tiles' global loads are in flight (16 bytes per lane) while one
+// is multiplied.  An operand that is contiguous along the contraction (K...) is stored as it is
+// loaded; one that is contiguous across it (the transposed factors of the weight gradients and of
+// the backward products) is loaded as 4 k x 8 rows per lane and turned in registers into eight
+// 8-byte k runs.  Each output is one accumulator chain over ascending k in steps of 16 (no split of
+// the contraction), so results equal gemm_kernel's bit for bit.  Bound: the latency of the k loop --
+// the shapes give each CU one or two blocks -- not the matrix cores.  Against gemm_kernel, which reads
+// two bytes per lane and load, 12 training steps (batch 1,024, 136-256-256-4,097) and one read of the
+// parameters went from 19.8 to 2.06 ms, with the loss and update kernels below.
+enum Along { ALONG_K, ALONG_ROW };  // what is contiguous in memory: the contraction, or the operand's rows
+
+struct TileArgs {
+    int M, N, K;
+    const uint16_t *A;
+    int lda;  // elements between rows (ALONG_K) or between k (ALONG_ROW)
+    const uint16_t *B;
+    int ldb;
+    float *C;  // float32 output or null
+    int ldc;
+    uint16_t *Cb;  // bf16 output or null
+    int ldcb;
+    const float *bias;     // per column, or null
+    const uint16_t *mask;  // zero the output where mask[m][n] <= 0 (ReLU backward), or null
+    int ldm;
+    int relu;
+    float *rowsum;  // sum over k of A per row m, ascending k (the bias gradient), or null
+    float *clear;   // two floats set to zero, or null
+};
+
+// BR rows x BK of one operand: global memory -> registers -> LDS
+template <int BR, int BK, Along AL> struct Stage {
+    static constexpr int LD = BK + 8;
+    static constexpr int UNITS = AL == ALONG_K ? BR * BK / 8 : BR * BK / 32;
+    static constexpr int PER = (UNITS + 255) / 256;  // units per thread
+    static constexpr int RW = AL == ALONG_K ? 1 : 4;
+    uint4 v[PER][RW];
+    // R rows exist; k runs to K.  Rows past R read a valid row (their outputs are not stored); k past
+    // K reads as zero
+    __device__ __forceinline__ void load(const uint16_t *X, int ld, int r0, int R, int k0, int K) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int u = (int)threadIdx.x + 256 * i;
+            if (UNITS % 256 != 0 && u >= UNITS) break;
+            if constexpr (AL == ALONG_K) {
+                const int r = min(r0 + u / (BK / 8), R - 1), k = k0 + (u % (BK / 8)) * 8;
+                v[i][0] = k < K ? *reinterpret_cast<const uint4 *>(X + (size_t)r * ld + k) : make_uint4(0u, 0u, 0u, 0u);
+                if (k < K && k + 8 > K) {
+                    uint32_t w[4] = {v[i][0].x, v[i][0].y, v[i][0].z, v[i][0].w};
+#pragma unroll
+                    for (int t = 0; t < 8; ++t)
+                        if (k + t >= K) w[t >> 1] &= (t & 1) ? 0x0000ffffu : 0xffff0000u;
+                    v[i][0] = make_uint4(w[0], w[1], w[2], w[3]);
+                }
+            } else {
+                const int r = min(r0 + (u % (BR / 8)) * 8, (R - 1) & ~7), k = k0 + (u / (BR / 8)) * 4;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    v[i][t] = k + t < K ? *reinterpret_cast<const uint4 *>(X + (size_t)(k + t) * ld + r)
+                                        : make_uint4(0u, 0u, 0u, 0u);
+            }
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t *lds) const {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int u = (int)threadIdx.x + 256 * i;
+            if (UNITS % 256 != 0 && u >= UNITS) break;
+            if constexpr (AL == ALONG_K) {
+                *reinterpret_cast<uint4 *>(lds + (u / (BK / 8)) * LD + (u % (BK / 8)) * 8) = v[i][0];
+            } else {
+                uint16_t *o = lds + (u % (BR / 8)) * 8 * LD + (u / (BR / 8)) * 4;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
+                    uint32_t w[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        w[j] = t < 2 ? v[i][j].x : t < 4 ? v[i][j].y : t < 6 ? v[i][j].z : v[i][j].w;
+                    uint2 x;
+                    x.x = __builtin_amdgcn_perm(w[1], w[0], sel);
+                    x.y = __builtin_amdgcn_perm(w[3], w[2], sel);
+                    *reinterpret_cast<uint2 *>(o + t * LD) = x;
+                }
+            }
+        }
+    }
+};
+
+template <int BM, int BN, int BK, Along AA, Along AB, int PF>
+__device__ __forceinline__ void tile_gemm(const TileArgs &g, int bm, int bn, uint16_t *lds) {
+    using SA = Stage<BM, BK, AA>;
+    using SB = Stage<BN, BK, AB>;
+    constexpr int LD = SA::LD, TM = BM / 32, TN = BN / 32, BUF = (BM + BN) * LD;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m0 = bm * BM, n0 = bn * BN;
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+    v4f acc[TM][TN];
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (g.clear && bm == 0 && bn == 0 && tid < 2) g.clear[tid] = 0.0f;
+    const bool sums = g.rowsum && bn == 0;
+    float rs = 0.0f;
+    SA sa[PF];
+    SB sb[PF];
+    const int nk = (g.K + BK - 1) / BK;
+    const auto fetch = [&](int slot, int it) {
+        if (it < nk) {
+            sa[slot].load(g.A, g.lda, m0, g.M, it * BK, g.K);
+            sb[slot].load(g.B, g.ldb, n0, g.N, it * BK, g.K);
+        }
+    };
+#pragma unroll
+    for (int p = 0; p < PF; ++p) fetch(p, p);
+    for (int it0 = 0; it0 < nk; it0 += PF) {
+#pragma unroll
+        for (int p = 0; p < PF; ++p) {
+            const int it = it0 + p;
+            if (it >= nk) break;
+            // two buffers and one barrier per tile: a wave that writes tile it + 1 has passed the barrier
+            // of tile it, so every wave is done with the buffer of tile it - 1
+            uint16_t *As = lds + (it & 1) * BUF, *Bs = As + BM * LD;
+            sa[p].store(As);
+            sb[p].store(Bs);
+            __syncthreads();
+            fetch(p, it + PF);
+#pragma unroll
+            for (int kk = 0; kk < BK; kk += 16) {
+                v4s a[TM], b[TN];
+#pragma unroll
+                for (int mi = 0; mi < TM; ++mi)
+                    a[mi] = *reinterpret_cast<const v4s *>(As + (wm + mi * 16 + (lane & 15)) * LD + kk + 4 * (lane >> 4));
+#pragma unroll
+                for (int ni = 0; ni < TN; ++ni)
+                    b[ni] = *reinterpret_cast<const v4s *>(Bs + (wn + ni * 16 + (lane & 15)) * LD + kk + 4 * (lane >> 4));
+#pragma unroll
+                for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+                    for (int ni = 0; ni < TN; ++ni)
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mi], b[ni], acc[mi][ni], 0, 0, 0);
+            }
+            if (sums && tid < BM) {
+#pragma unroll
+                for (int k = 0; k < BK; k += 8) {
+                    const uint4 x = *reinterpret_cast<const uint4 *>(As + tid * LD + k);
+                    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        rs += __uint_as_float(w[t] << 16);
+                        rs += __uint_as_float(w[t] & 0xffff0000u);
+                    }
+                }
+            }
+        }
+    }
+    if (sums && tid < BM && m0 + tid < g.M) g.rowsum[m0 + tid] = rs;
+#pragma unroll
+    for (int mi = 0; mi < TM; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int m = m0 + wm + mi * 16 + 4 * (lane >> 4) + j;
+                const int n = n0 + wn + ni * 16 + (lane & 15);
                 if (m < g.M && n < g.N) {
-                    float v = g.alpha * acc[mi][ni][j];
+                    float v = acc[mi][ni][j];
                     if (g.bias) v += g.bias[n];
                     if (g.relu) v = fmaxf(v, 0.0f);
-                    if (g.mask && bf2f(g.mask[(long long)m * g.ldm + n]) <= 0.0f) v = 0.0f;
-                    if (g.C) g.C[(long long)m * g.ldc + n] = v;
-                    if (g.Cb) g.Cb[(long long)m * g.ldcb + n] = f2bf(v);
+                    if (g.mask && bf2f(g.mask[(size_t)m * g.ldm + n]) <= 0.0f) v = 0.0f;
+                    if (g.C) g.C[(size_t)m * g.ldc + n] = v;
+                    if (g.Cb) g.Cb[(size_t)m * g.ldcb + n] = f2bf(v);
                 }
             }
 }
 
-static int gemm(const GemmArgs &g, hipStream_t st) {
-    if (g.M <= 0 || g.N <= 0 || g.K <= 0) return 0;
-    dim3 grid((g.N + GBN - 1) / GBN, (g.M + GBM - 1) / GBM);
-    hipLaunchKernelGGL(gemm_kernel, grid, dim3(256), 0, st, g);
+template <int BM, int BN, int BK, Along AA, Along AB, int PF>
+__global__ __launch_bounds__(256) void tile_kernel(TileArgs g) {
+    __shared__ __align__(16) uint16_t lds[2 * (BM + BN) * (BK + 8)];
+    tile_gemm<BM, BN, BK, AA, AB, PF>(g, blockIdx.y, blockIdx.x, lds);
+}
+
+// Two independent products of one backward stage in one launch, blocks of the first before those of
+// the second: the input gradient (rows along k, weights across it) and the weight gradient (both
+// across it).  Neither fills the device alone.
+template <int BM1, int BN1, int BK1, int PF1, int BM2, int BN2, int BK2, int PF2>
+__global__ __launch_bounds__(256) void tile_pair_kernel(TileArgs g1, int nb1, int nn1, TileArgs g2, int nn2) {
+    constexpr int L1 = 2 * (BM1 + BN1) * (BK1 + 8), L2 = 2 * (BM2 + BN2) * (BK2 + 8);
+    __shared__ __align__(16) uint16_t lds[L1 > L2 ? L1 : L2];
+    const int b = blockIdx.x;
+    if (b < nb1)
+        tile_gemm<BM1, BN1, BK1, ALONG_K, ALONG_ROW, PF1>(g1, b / nn1, b % nn1, lds);
+    else
+        tile_gemm<BM2, BN2, BK2, ALONG_ROW, ALONG_ROW, PF2>(g2, (b - nb1) / nn2, (b - nb1) % nn2, lds);
+}
+
+static int tiles(int n, int b) { return (n + b - 1) / b; }
+
+template <int BM, int BN, int BK, Along AA, Along AB, int PF>
+static int tile_launch(const TileArgs &g, hipStream_t st) {
+    hipLaunchKernelGGL((tile_kernel<BM, BN, BK, AA, AB, PF>), dim3(tiles(g.N, BN), tiles(g.M, BM)), dim3(256), 0, st, g);
     MHIP(hipGetLastError());
     return 0;
 }
 
-static GemmArgs gemm_args(int M, int N, int K, const uint16_t *A, long long sam, long long sak, const uint16_t *B,
-                          long long sbk, long long sbn) {
-    GemmArgs g{};
-    g.M = M;
-    g.N = N;
-    g.K = K;
-    g.A = A;
-    g.sam = sam;
-    g.sak = sak;
-    g.B = B;
-    g.sbk = sbk;
-    g.sbn = sbn;
-    g.alpha = 1.0f;
-    return g;
-}
-
 extern "C" int song_gemm_bf16(int M, int N, int K, const uint16_t *d_a, int sam, int sak, const uint16_t *d_b, int sbk,
                               int sbn, float *d_c, int ldc, float alpha, void *stream) {
-    GemmArgs g = gemm_args(M, N, K, d_a, sam, sak, d_b, sbk, sbn);
-    g.C = d_c;
-    g.ldc = ldc;
-    g.alpha = alpha;
-    return gemm(g, (hipStream_t)stream);
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const GemmArgs g{M, N, K, d_a, sam, sak, d_b, sbk, sbn, d_c, ldc, alpha};
+    hipLaunchKernelGGL(gemm_kernel, dim3(tiles(N, GBN), tiles(M, GBM)), dim3(256), 0, (hipStream_t)stream, g);
+    MHIP(hipGetLastError());
+    return 0;
 }
 
 // ---------------------------------------------------------------- loss, sums, Adam
 
-// One 64-lane block per row: softmax cross-entropy over the first C logits against the
-// label, squared error of logit C against the stop target; writes dZ (bf16) and adds the
-// batch means of both losses to loss[0..1].
-__global__ __launch_bounds__(64) void loss_kernel(const float *Z, int ldz, int C, const int *labels, const float *stop_t,
-                                                  int B, float stop_w, uint16_t *dZ, int lddz, float *loss) {
-    const int row = blockIdx.x, lane = threadIdx.x;
+// One block of four waves per row: softmax cross-entropy over the first C logits against the label,
+// squared error of logit C against the stop target; writes dZ (bf16) and adds the batch means of both
+// losses to loss[0..1].  Every exponential is computed once, by all waves, and kept in LDS (C + 1
+// floats); the first wave adds them, lane l the columns l, l + 64, ... in ascending order and then
+// the lanes in halving steps, the order a single wave per row has, so the sum does not depend on the
+// waves.  Rows too wide for LDS (IN_LDS false) compute the exponentials again where they are used.
+// One wave per row that computed each exponential twice took 64 us for 1,024 rows of 4,097.
+constexpr int LOSS_LDS_CLASSES = 12288;  // 48 KB: three blocks fit a CU's LDS
+template <bool IN_LDS>
+__global__ __launch_bounds__(256) void loss_kernel(const float *Z, int ldz, int C, const int *labels, const float *stop_t,
+                                                   int B, float stop_w, uint16_t *dZ, int lddz, float *loss) {
+    extern __shared__ __align__(16) float ex[];
+    __shared__ float red[8];
+    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float *z = Z + (long long)row * ldz;
     float mx = -INFINITY;
-    for (int c = lane; c < C; c += 64) mx = fmaxf(mx, z[c]);
+    for (int c = tid; c < C; c += 256) {
+        const float v = z[c];
+        if (IN_LDS) ex[c] = v;
+        mx = fmaxf(mx, v);
+    }
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    float se = 0.0f;
-    for (int c = lane; c < C; c += 64) se += expf(z[c] - mx);
-    for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o);
+    if (lane == 0) red[wave] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if (IN_LDS) {
+        for (int c = tid; c < C; c += 256) ex[c] = expf(ex[c] - mx);
+        __syncthreads();
+    }
+    if (wave == 0) {
+        float se = 0.0f;
+        for (int c = lane; c < C; c += 64) se += IN_LDS ? ex[c] : expf(z[c] - mx);
+        for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o);
+        if (lane == 0) red[4] = se;
+    }
+    __syncthreads();
+    const float se = red[4];
     const int lab = labels[row];
     const float inv = 1.0f / (float)B;
-    for (int c = lane; c < C; c += 64) {
-        const float p = expf(z[c] - mx) / se;
+    for (int c = tid; c < C; c += 256) {
+        const float p = (IN_LDS ? ex[c] : expf(z[c] - mx)) / se;
         dZ[(long long)row * lddz + c] = f2bf((p - (c == lab ? 1.0f : 0.0f)) * inv);
     }
-    if (lane == 0) {
+    if (tid == 0) {
         const float diff = z[C] - stop_t[row];
         dZ[(long long)row * lddz + C] = f2bf(2.0f * stop_w * diff * inv);
         atomicAdd(&loss[0], (logf(se) + mx - z[lab]) * inv);
@@ -187,30 +384,78 @@ __global__ __launch_bounds__(64) void loss_kernel(const float *Z, int ldz, int C
     }
 }
 
-// out[n] = sum over rows of G[m][n] (bf16 rows)
-__global__ void colsum_kernel(const uint16_t *G, int M, int N, int ldg, float *out) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    float s = 0.0f;
-    for (int m = 0; m < M; ++m) s += bf2f(G[(long long)m * ldg + n]);
-    out[n] = s;
+// The parameter vector's segments (W1 b1 W2 b2 W3 b3) and the bf16 copies of its weights
+struct ParamCopies {
+    long long off[6], cnt[6];
+    uint16_t *Wb[3];
+    uint16_t *W3i;  // the output weights in the layout infer_kernel reads (see refresh_kernel)
+    int rows3, hidden, npad;
+};
+struct AdamArgs {
+    float *p;
+    const float *g;
+    float *m, *v;
+    float lr, b1, b2, c1, c2, eps;
+};
+
+__device__ __forceinline__ void adam_one(const AdamArgs &a, float gi, float &p, float &m, float &v) {
+    // contracted as written (the compiler would choose per use, and the two loops would differ)
+    m = fmaf(1.0f - a.b1, gi, a.b1 * m);
+    v = fmaf(gi, (1.0f - a.b2) * gi, a.b2 * v);
+    p -= a.lr * (m / a.c1) / (sqrtf(v / a.c2) + a.eps);
 }
 
-__global__ void adam_kernel(float *p, const float *g, float *m, float *v, long long n, float lr, float b1, float b2,
-                            float c1, float c2, float eps) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-__global__ void to_bf16_kernel(const float *x, uint16_t *y, long long n) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = f2bf(x[i]);
+// Every parameter once: with ADAM the update, then the bf16 copies of the weights, the output
+// weights twice -- row by row for the products, and for inference in k quads: fragment (k-step s,
+// k-quad q, column n) = W3[n][16s + 4q .. +4) at W3i[((4s + q) * npad + n) * 4], zero for n >= rows3,
+// so that the 16 columns a lane group reads per step are one aligned 128-byte run.  The first blocks
+// take W3 in tiles of 16 rows x 64 columns, four columns per lane (64-byte runs of the float arrays,
+// 128-byte runs of W3i); the rest take the other segments in order.  Bound by memory: 30 bytes per
+// parameter.  As five kernels (update, three conversions, interleave) a step took 26 us at 1.16
+// million parameters and read the new weights three times.
+template <bool ADAM>
+__global__ __launch_bounds__(256) void refresh_kernel(AdamArgs a, ParamCopies c, int w3_blocks) {
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x < w3_blocks) {
+        const int kt = (c.hidden + 63) / 64;
+        const int n = ((int)blockIdx.x / kt) * 16 + (tid & 15), k = ((int)blockIdx.x % kt) * 64 + (tid >> 4) * 4;
+        if (k >= c.hidden) return;
+        uint16_t h[4] = {0, 0, 0, 0};
+        if (n < c.rows3) {
+            const long long i = c.off[4] + (long long)n * c.hidden + k;  // (a multiple of four: so are all segments)
+            float4 p = *reinterpret_cast<const float4 *>(a.p + i);
+            if constexpr (ADAM) {
+                const float4 gr = *reinterpret_cast<const float4 *>(a.g + i);
+                float4 mo = *reinterpret_cast<const float4 *>(a.m + i), vo = *reinterpret_cast<const float4 *>(a.v + i);
+                adam_one(a, gr.x, p.x, mo.x, vo.x);
+                adam_one(a, gr.y, p.y, mo.y, vo.y);
+                adam_one(a, gr.z, p.z, mo.z, vo.z);
+                adam_one(a, gr.w, p.w, mo.w, vo.w);
+                *reinterpret_cast<float4 *>(a.p + i) = p;
+                *reinterpret_cast<float4 *>(a.m + i) = mo;
+                *reinterpret_cast<float4 *>(a.v + i) = vo;
+            }
+            h[0] = f2bf(p.x), h[1] = f2bf(p.y), h[2] = f2bf(p.z), h[3] = f2bf(p.w);
+            *reinterpret_cast<ushort4 *>(c.Wb[2] + (long long)n * c.hidden + k) = make_ushort4(h[0], h[1], h[2], h[3]);
+        }
+        *reinterpret_cast<ushort4 *>(c.W3i + ((long long)(k >> 2) * c.npad + n) * 4) = make_ushort4(h[0], h[1], h[2], h[3]);
+        return;
+    }
+    // W1 b1 W2 b2 are one run, b3 is the last
+    const long long run = c.off[4];
+    long long i = ((long long)blockIdx.x - w3_blocks) * 256 + tid;
+    if (i >= run) i += c.cnt[4];
+    if (i >= c.off[5] + c.cnt[5]) return;
+    float p = a.p[i];
+    if constexpr (ADAM) {
+        float mo = a.m[i], vo = a.v[i];
+        adam_one(a, a.g[i], p, mo, vo);
+        a.p[i] = p;
+        a.m[i] = mo;
+        a.v[i] = vo;
+    }
+    if (i < c.cnt[0]) c.Wb[0][i] = f2bf(p);
+    else if (i >= c.off[2] && i < c.off[2] + c.cnt[2]) c.Wb[1][i - c.off[2]] = f2bf(p);
 }
 
 // ---------------------------------------------------------------- features
@@ -329,7 +574,7 @@ __device__ __forceinline__ void tile_layer(const uint16_t *in, int ldin, int K, 
     }
 }
 
-// As tile_layer, with the weights in the k-quad interleaved layout (interleave_kernel): a lane
+// As tile_layer, with the weights in the k-quad interleaved layout (refresh_kernel): a lane
 // group's 16 fragments of one step are one contiguous 128-byte run (four full cache lines per
 // load instead of 32 bytes of sixteen).  The lanes take the same k as in tile_layer, so the
 // accumulators are identical.
@@ -579,8 +824,10 @@ struct song_mlp {
     uint16_t *Wb[3] = {nullptr, nullptr, nullptr};
     uint16_t *W3i = nullptr;  // inference copy of the output weights, k-quad interleaved (infer_kernel)
     int npad = 0;             // its column count: C + 1 rounded up to 16
+    int ldz = 0;              // row stride of Z and dZ: C + 1 rounded up to 8 (16-byte rows)
     uint16_t *H1 = nullptr, *H2 = nullptr, *dZ = nullptr, *dH2 = nullptr, *dH1 = nullptr;
     float *Z = nullptr, *loss = nullptr;
+    uint16_t *Xa = nullptr;  // aligned copy of inputs that are not
     int t = 0;
 };
 
@@ -591,31 +838,27 @@ static uint64_t splitmix(uint64_t &s) {
     return z ^ (z >> 31);
 }
 
-// The output weights W [N][K] (bf16, row-major) in the layout the inference GEMM reads: fragment
-// (k-step s, k-quad q, column n) = W[n][16s + 4q .. +4) at Wi[((4s + q) * npad + n) * 4], zero for
-// n >= N, so the 16 columns one lane group reads per step are one aligned 128-byte run.
-__global__ __launch_bounds__(256) void interleave_kernel(const uint16_t *W, uint16_t *Wi, int N, int K, int npad) {
-    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (long long)K * npad) return;
-    const int t = (int)(e & 3);
-    const long long g = e >> 2;
-    const int n = (int)(g % npad);
-    const int sq = (int)(g / npad);
-    const int k = 16 * (sq >> 2) + 4 * (sq & 3) + t;
-    Wi[e] = n < N ? W[(long long)n * K + k] : (uint16_t)0;
-}
-
-static int refresh_bf16(song_mlp *m, hipStream_t st) {
-    for (int l = 0; l < 3; ++l) {
-        const long long n = m->cnt[2 * l];
-        hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m->P + m->off[2 * l],
-                           m->Wb[l], n);
+template <bool ADAM> static int refresh(song_mlp *m, AdamArgs a, hipStream_t st) {
+    ParamCopies c{};
+    for (int i = 0; i < 6; ++i) {
+        c.off[i] = m->off[i];
+        c.cnt[i] = m->cnt[i];
     }
-    const long long ni = (long long)m->hidden * m->npad;
-    hipLaunchKernelGGL(interleave_kernel, dim3((unsigned)((ni + 255) / 256)), dim3(256), 0, st, m->Wb[2], m->W3i,
-                       m->C + 1, m->hidden, m->npad);
+    for (int l = 0; l < 3; ++l) c.Wb[l] = m->Wb[l];
+    c.W3i = m->W3i;
+    c.rows3 = m->C + 1;
+    c.hidden = m->hidden;
+    c.npad = m->npad;
+    const int w3 = (m->npad / 16) * ((m->hidden + 63) / 64);
+    const long long rest = m->total - m->cnt[4];
+    hipLaunchKernelGGL(refresh_kernel<ADAM>, dim3((unsigned)(w3 + (rest + 255) / 256)), dim3(256), 0, st, a, c, w3);
     MHIP(hipGetLastError());
     return 0;
+}
+static int refresh_bf16(song_mlp *m, hipStream_t st) {
+    AdamArgs a{};
+    a.p = m->P;
+    return refresh<false>(m, a, st);
 }
 
 extern "C" int song_mlp_create(int in_dim, int hidden, int n_classes, int max_batch, uint64_t seed, song_mlp **out) {
@@ -659,10 +902,11 @@ extern "C" int song_mlp_create(int in_dim, int hidden, int n_classes, int max_ba
         if (hipMalloc(&m->Wb[l], m->cnt[2 * l] * 2)) return bad("bf16 weights");
     m->npad = (n_classes + 1 + 15) & ~15;
     if (hipMalloc(&m->W3i, (size_t)m->npad * hidden * 2)) return bad("interleaved output weights");
-    const long long B = max_batch, NO = n_classes + 1;
-    if (hipMalloc(&m->H1, B * hidden * 2) || hipMalloc(&m->H2, B * hidden * 2) || hipMalloc(&m->dZ, B * NO * 2) ||
-        hipMalloc(&m->dH2, B * hidden * 2) || hipMalloc(&m->dH1, B * hidden * 2) || hipMalloc(&m->Z, B * NO * 4) ||
-        hipMalloc(&m->loss, 8))
+    m->ldz = (n_classes + 1 + 7) & ~7;
+    const long long B = max_batch, LZ = m->ldz;
+    if (hipMalloc(&m->H1, B * hidden * 2) || hipMalloc(&m->H2, B * hidden * 2) || hipMalloc(&m->dZ, B * LZ * 2) ||
+        hipMalloc(&m->dH2, B * hidden * 2) || hipMalloc(&m->dH1, B * hidden * 2) || hipMalloc(&m->Z, B * LZ * 4) ||
+        hipMalloc(&m->loss, 8) || hipMalloc(&m->Xa, B * m->width * 2))
         return bad("activations");
     if (hipMemcpy(m->P, init.data(), o * 4, hipMemcpyHostToDevice) || hipMemset(m->Mo, 0, o * 4) ||
         hipMemset(m->Vo, 0, o * 4) || hipMemset(m->G, 0, o * 4)) {
@@ -680,7 +924,7 @@ extern "C" int song_mlp_create(int in_dim, int hidden, int n_classes, int max_ba
 extern "C" int song_mlp_destroy(song_mlp *m) {
     if (!m) return 0;
     void *ptrs[] = {m->P, m->G, m->Mo, m->Vo, m->Wb[0], m->Wb[1], m->Wb[2], m->W3i, m->H1, m->H2, m->dZ, m->dH2,
-                    m->dH1, m->Z, m->loss};
+                    m->dH1, m->Z, m->loss, m->Xa};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     delete m;
@@ -714,61 +958,85 @@ extern "C" int song_mlp_loss_grad(song_mlp *m, const uint16_t *d_x, const int *d
     if (!m || !d_x || !d_labels || !d_stop) return mfail(-1, "null argument");
     if (batch < 1 || batch > m->max_batch) return mfail(-1, "batch %d outside [1, %d]", batch, m->max_batch);
     hipStream_t st = (hipStream_t)stream;
-    const int W = m->width, Hd = m->hidden, NO = m->C + 1;
-    float *W1 = m->P + m->off[0], *b1 = m->P + m->off[1], *b2 = m->P + m->off[3], *b3 = m->P + m->off[5];
-    (void)W1;
-    // forward
-    GemmArgs g = gemm_args(batch, Hd, W, d_x, W, 1, m->Wb[0], 1, W);
+    const int W = m->width, Hd = m->hidden, NO = m->C + 1, LZ = m->ldz;
+    float *b1 = m->P + m->off[1], *b2 = m->P + m->off[3], *b3 = m->P + m->off[5], *G = m->G;
+    // the tile kernels read the inputs in 16-byte units; the network's own buffers are aligned
+    const uint16_t *x = d_x;
+    if (((uintptr_t)d_x & 15) != 0) {
+        MHIP(hipMemcpyAsync(m->Xa, d_x, (size_t)batch * W * 2, hipMemcpyDeviceToDevice, st));
+        x = m->Xa;
+    }
+    const auto args = [](int M, int N, int K, const uint16_t *A, int lda, const uint16_t *B, int ldb) {
+        TileArgs g{};
+        g.M = M;
+        g.N = N;
+        g.K = K;
+        g.A = A;
+        g.lda = lda;
+        g.B = B;
+        g.ldb = ldb;
+        return g;
+    };
+    // forward: H1 = relu(X W1^T + b1), H2 = relu(H1 W2^T + b2), Z = H2 W3^T + b3
+    TileArgs g = args(batch, Hd, W, x, W, m->Wb[0], W);
     g.Cb = m->H1;
     g.ldcb = Hd;
     g.bias = b1;
     g.relu = 1;
-    if (gemm(g, st)) return -2;
-    g = gemm_args(batch, Hd, Hd, m->H1, Hd, 1, m->Wb[1], 1, Hd);
+    g.clear = m->loss;
+    if (tile_launch<32, 32, 64, ALONG_K, ALONG_K, 2>(g, st)) return -2;
+    g = args(batch, Hd, Hd, m->H1, Hd, m->Wb[1], Hd);
     g.Cb = m->H2;
     g.ldcb = Hd;
     g.bias = b2;
     g.relu = 1;
-    if (gemm(g, st)) return -2;
-    g = gemm_args(batch, NO, Hd, m->H2, Hd, 1, m->Wb[2], 1, Hd);
+    if (tile_launch<32, 32, 64, ALONG_K, ALONG_K, 2>(g, st)) return -2;
+    g = args(batch, NO, Hd, m->H2, Hd, m->Wb[2], Hd);
     g.C = m->Z;
-    g.ldc = NO;
+    g.ldc = LZ;
     g.bias = b3;
-    if (gemm(g, st)) return -2;
-    MHIP(hipMemsetAsync(m->loss, 0, 8, st));
-    hipLaunchKernelGGL(loss_kernel, dim3(batch), dim3(64), 0, st, m->Z, NO, m->C, d_labels, d_stop, batch, stop_weight,
-                       m->dZ, NO, m->loss);
+    if (tile_launch<64, 64, 64, ALONG_K, ALONG_K, 2>(g, st)) return -2;
+    const bool in_lds = m->C <= LOSS_LDS_CLASSES;
+    hipLaunchKernelGGL(in_lds ? loss_kernel<true> : loss_kernel<false>, dim3(batch), dim3(256),
+                       in_lds ? (size_t)m->C * sizeof(float) : 0, st, m->Z, LZ, m->C, d_labels, d_stop, batch,
+                       stop_weight, m->dZ, LZ, m->loss);
     MHIP(hipGetLastError());
-    // backward: dW3 = dZ^T H2, db3, dH2 = dZ W3 * (H2 > 0), ...
-    float *G = m->G;
-    g = gemm_args(NO, Hd, batch, m->dZ, 1, NO, m->H2, Hd, 1);
-    g.C = G + m->off[4];
-    g.ldc = Hd;
-    if (gemm(g, st)) return -2;
-    hipLaunchKernelGGL(colsum_kernel, dim3((NO + 255) / 256), dim3(256), 0, st, m->dZ, batch, NO, NO, G + m->off[5]);
-    g = gemm_args(batch, Hd, NO, m->dZ, NO, 1, m->Wb[2], Hd, 1);
-    g.Cb = m->dH2;
-    g.ldcb = Hd;
-    g.mask = m->H2;
-    g.ldm = Hd;
-    if (gemm(g, st)) return -2;
-    g = gemm_args(Hd, Hd, batch, m->dH2, 1, Hd, m->H1, Hd, 1);
-    g.C = G + m->off[2];
-    g.ldc = Hd;
-    if (gemm(g, st)) return -2;
-    hipLaunchKernelGGL(colsum_kernel, dim3((Hd + 255) / 256), dim3(256), 0, st, m->dH2, batch, Hd, Hd, G + m->off[3]);
-    g = gemm_args(batch, Hd, Hd, m->dH2, Hd, 1, m->Wb[1], Hd, 1);
-    g.Cb = m->dH1;
-    g.ldcb = Hd;
-    g.mask = m->H1;
-    g.ldm = Hd;
-    if (gemm(g, st)) return -2;
-    g = gemm_args(Hd, W, batch, m->dH1, 1, Hd, d_x, W, 1);
+    // backward: dH2 = dZ W3 * (H2 > 0) beside dW3 = dZ^T H2 and db3, then dH1 beside dW2 and db2, then dW1
+    TileArgs gi = args(batch, Hd, NO, m->dZ, LZ, m->Wb[2], Hd);
+    gi.Cb = m->dH2;
+    gi.ldcb = Hd;
+    gi.mask = m->H2;
+    gi.ldm = Hd;
+    TileArgs gw = args(NO, Hd, batch, m->dZ, LZ, m->H2, Hd);
+    gw.C = G + m->off[4];
+    gw.ldc = Hd;
+    gw.rowsum = G + m->off[5];
+    {
+        const int nb1 = tiles(batch, 32) * tiles(Hd, 32), nb2 = tiles(NO, 64) * tiles(Hd, 64);
+        hipLaunchKernelGGL((tile_pair_kernel<32, 32, 128, 2, 64, 64, 32, 2>), dim3(nb1 + nb2), dim3(256), 0, st, gi, nb1,
+                           tiles(Hd, 32), gw, tiles(Hd, 64));
+        MHIP(hipGetLastError());
+    }
+    gi = args(batch, Hd, Hd, m->dH2, Hd, m->Wb[1], Hd);
+    gi.Cb = m->dH1;
+    gi.ldcb = Hd;
+    gi.mask = m->H1;
+    gi.ldm = Hd;
+    gw = args(Hd, Hd, batch, m->dH2, Hd, m->H1, Hd);
+    gw.C = G + m->off[2];
+    gw.ldc = Hd;
+    gw.rowsum = G + m->off[3];
+    {
+        const int nb1 = tiles(batch, 32) * tiles(Hd, 32), nb2 = tiles(Hd, 32) * tiles(Hd, 32);
+        hipLaunchKernelGGL((tile_pair_kernel<32, 32, 64, 2, 32, 32, 64, 2>), dim3(nb1 + nb2), dim3(256), 0, st, gi, nb1,
+                           tiles(Hd, 32), gw, tiles(Hd, 32));
+        MHIP(hipGetLastError());
+    }
+    g = args(Hd, W, batch, m->dH1, Hd, x, W);
     g.C = G + m->off[0];
     g.ldc = W;
-    if (gemm(g, st)) return -2;
-    hipLaunchKernelGGL(colsum_kernel, dim3((Hd + 255) / 256), dim3(256), 0, st, m->dH1, batch, Hd, Hd, G + m->off[1]);
-    MHIP(hipGetLastError());
+    g.rowsum = G + m->off[1];
+    if (tile_launch<32, 32, 64, ALONG_ROW, ALONG_ROW, 2>(g, st)) return -2;
     if (loss_out) {
         MHIP(hipMemcpyAsync(loss_out, m->loss, 8, hipMemcpyDeviceToHost, st));
         MHIP(hipStreamSynchronize(st));
@@ -786,10 +1054,7 @@ extern "C" int song_mlp_adam_step(song_mlp *m, float lr, void *stream) {
     m->t += 1;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.0f - std::pow(b1, (float)m->t), c2 = 1.0f - std::pow(b2, (float)m->t);
-    hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((m->total + 255) / 256)), dim3(256), 0, st, m->P, m->G, m->Mo,
-                       m->Vo, m->total, lr, b1, b2, c1, c2, 1e-8f);
-    MHIP(hipGetLastError());
-    return refresh_bf16(m, st);
+    return refresh<true>(m, AdamArgs{m->P, m->G, m->Mo, m->Vo, lr, b1, b2, c1, c2, 1e-8f}, st);
 }
 
 extern "C" int song_mlp_infer(song_mlp *m, const uint16_t *d_x, int batch, int *d_top2, float *d_conf, float *d_stop,
