@@ -117,15 +117,14 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
 
 // The training products: operands whose rows are 16-byte aligned along one of their two directions.
 // A block computes BM x BN with 2 x 2 waves, BK of the contraction at a time, through two LDS buffers
-// of k-contiguous rows; the next PF tiles' global loads are in flight (16 bytes per lane) while one
-// is multiplied.  An operand that is contiguous along the contraction (K...) is stored as it is
-// loaded; one that is contiguous across it (the transposed factors of the weight gradients and of
-// the backward products) is loaded as 4 k x 8 rows per lane and turned in registers into eight
-// 8-byte k runs.  Each output is one accumulator chain over ascending k in steps of 16 (no split of
+// of k-contiguous rows; the next PF tiles' global loads are in flight while one is multiplied.  An
+// operand that is contiguous along the contraction is stored as it is loaded; one that is contiguous
+// across it (the transposed factors of the weight gradients and of the backward products) is turned
+// in registers (Stage).  Each output is one accumulator chain over ascending k in steps of 16 (no split of
 // the contraction), so results equal gemm_kernel's bit for bit.  Bound: the latency of the k loop --
 // the shapes give each CU one or two blocks -- not the matrix cores.  Against gemm_kernel, which reads
 // two bytes per lane and load, 12 training steps (batch 1,024, 136-256-256-4,097) and one read of the
-// parameters went from 19.8 to 2.06 ms, with the loss and update kernels below.
+// parameters went from 19.8 to 1.37 ms, with the loss and update kernels below.
 enum Along { ALONG_K, ALONG_ROW };  // what is contiguous in memory: the contraction, or the operand's rows
 
 struct TileArgs {
@@ -143,62 +142,104 @@ struct TileArgs {
     int ldm;
     int relu;
     float *rowsum;  // sum over k of A per row m, ascending k (the bias gradient), or null
-    float *clear;   // two floats set to zero, or null
 };
 
-// BR rows x BK of one operand: global memory -> registers -> LDS
+// BR rows x BK of one operand, by 128 threads (t = 0..127): global memory -> registers -> LDS.  A unit
+// is 8 k of one row (ALONG_K, one 16-byte load) or 4 k of 4 rows (ALONG_ROW, four 8-byte loads turned
+// into four 8-byte k runs).  Each unit keeps its pointer and advances by a tile, so a load costs no
+// address arithmetic; k past K (the last tile only) reads as zero; rows past R read a valid row,
+// whose outputs are not stored.
+// The two operands' movers share one state (Mover): half the block's waves run one, half the other.
+template <int NP> struct Mover {
+    const uint16_t *ptr[NP];
+    size_t ld, step;
+    int t;
+};
 template <int BR, int BK, Along AL> struct Stage {
-    static constexpr int LD = BK + 8;
-    static constexpr int UNITS = AL == ALONG_K ? BR * BK / 8 : BR * BK / 32;
-    static constexpr int PER = (UNITS + 255) / 256;  // units per thread
-    static constexpr int RW = AL == ALONG_K ? 1 : 4;
-    uint4 v[PER][RW];
-    // R rows exist; k runs to K.  Rows past R read a valid row (their outputs are not stored); k past
-    // K reads as zero
-    __device__ __forceinline__ void load(const uint16_t *X, int ld, int r0, int R, int k0, int K) {
+    // LDS row stride: 2 words more than a multiple of 32, so that the 16 rows of a fragment read, and
+    // the 4 x 4 units that 16 lanes of a turned store write, fall on different banks (a stride of BK + 8
+    // elements had 14 of 22 LDS cycles per access in conflicts, and LDS was what bound the backward)
+    static constexpr int LD = BK + 4;
+    static constexpr int UNITS = AL == ALONG_K ? BR * BK / 8 : BR * BK / 16;
+    static constexpr int PER = UNITS / 128;              // units per thread
+    static constexpr int REGS = AL == ALONG_K ? PER : 2 * PER;  // 16-byte registers per tile
+    static_assert(UNITS % 128 == 0, "whole units per thread");
+    // 16 lanes of turned units take 4 row groups x 4 k groups
+    __device__ __forceinline__ static int row_of(int u) {
+        return AL == ALONG_K ? u / (BK / 8) : (((u >> 4) % (BR / 16)) * 4 + (u & 3)) * 4;
+    }
+    __device__ __forceinline__ static int k_of(int u) {
+        return AL == ALONG_K ? (u % (BK / 8)) * 8 : (((u >> 4) / (BR / 16)) * 4 + ((u >> 2) & 3)) * 4;
+    }
+    template <int NP>
+    __device__ __forceinline__ static void init(Mover<NP> &c, const uint16_t *X, int ldx, int r0, int R) {
+        const size_t ld = (size_t)ldx;
+        c.ld = ld;
+        c.step = AL == ALONG_K ? (size_t)BK : (size_t)BK * ld;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int u = (int)threadIdx.x + 256 * i;
-            if (UNITS % 256 != 0 && u >= UNITS) break;
-            if constexpr (AL == ALONG_K) {
-                const int r = min(r0 + u / (BK / 8), R - 1), k = k0 + (u % (BK / 8)) * 8;
-                v[i][0] = k < K ? *reinterpret_cast<const uint4 *>(X + (size_t)r * ld + k) : make_uint4(0u, 0u, 0u, 0u);
-                if (k < K && k + 8 > K) {
-                    uint32_t w[4] = {v[i][0].x, v[i][0].y, v[i][0].z, v[i][0].w};
+            const int u = c.t + 128 * i;
+            const int r = AL == ALONG_K ? min(r0 + row_of(u), R - 1) : min(r0 + row_of(u), (R - 1) & ~3);
+            c.ptr[i] = AL == ALONG_K ? X + (size_t)r * ld + k_of(u) : X + (size_t)k_of(u) * ld + r;
+        }
+    }
+    // the tile the pointers stand at (its first k is k0)
+    template <int NP, int NV> __device__ __forceinline__ static void load(Mover<NP> &c, uint4 (&v)[NV], int k0, int K) {
+        const size_t ld = c.ld;
+        if (k0 + BK <= K) {
 #pragma unroll
-                    for (int t = 0; t < 8; ++t)
-                        if (k + t >= K) w[t >> 1] &= (t & 1) ? 0x0000ffffu : 0xffff0000u;
-                    v[i][0] = make_uint4(w[0], w[1], w[2], w[3]);
+            for (int i = 0; i < PER; ++i) {
+                if constexpr (AL == ALONG_K) {
+                    v[i] = *reinterpret_cast<const uint4 *>(c.ptr[i]);
+                } else {
+                    const uint2 a = *reinterpret_cast<const uint2 *>(c.ptr[i]);
+                    const uint2 b = *reinterpret_cast<const uint2 *>(c.ptr[i] + ld);
+                    const uint2 e = *reinterpret_cast<const uint2 *>(c.ptr[i] + 2 * ld);
+                    const uint2 d = *reinterpret_cast<const uint2 *>(c.ptr[i] + 3 * ld);
+                    v[2 * i] = make_uint4(a.x, a.y, b.x, b.y);
+                    v[2 * i + 1] = make_uint4(e.x, e.y, d.x, d.y);
                 }
-            } else {
-                const int r = min(r0 + (u % (BR / 8)) * 8, (R - 1) & ~7), k = k0 + (u / (BR / 8)) * 4;
+            }
+        } else {
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    v[i][t] = k + t < K ? *reinterpret_cast<const uint4 *>(X + (size_t)(k + t) * ld + r)
-                                        : make_uint4(0u, 0u, 0u, 0u);
+            for (int i = 0; i < PER; ++i) {
+                const int k = k0 + k_of(c.t + 128 * i);
+                if constexpr (AL == ALONG_K) {
+                    v[i] = k < K ? *reinterpret_cast<const uint4 *>(c.ptr[i]) : make_uint4(0u, 0u, 0u, 0u);
+                    const auto cut = [&](uint32_t w, int e) {  // elements e, e + 1 of the unit
+                        return (k + e < K ? w & 0x0000ffffu : 0u) | (k + e + 1 < K ? w & 0xffff0000u : 0u);
+                    };
+                    v[i] = make_uint4(cut(v[i].x, 0), cut(v[i].y, 2), cut(v[i].z, 4), cut(v[i].w, 6));
+                } else {
+                    const auto one = [&](int j) {
+                        return k + j < K ? *reinterpret_cast<const uint2 *>(c.ptr[i] + j * ld) : make_uint2(0u, 0u);
+                    };
+                    const uint2 a = one(0), b = one(1), e = one(2), d = one(3);
+                    v[2 * i] = make_uint4(a.x, a.y, b.x, b.y);
+                    v[2 * i + 1] = make_uint4(e.x, e.y, d.x, d.y);
+                }
             }
         }
     }
-    __device__ __forceinline__ void store(uint16_t *lds) const {
+    template <int NP, int NV>
+    __device__ __forceinline__ static void store(const Mover<NP> &c, const uint4 (&v)[NV], uint16_t *lds) {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int u = (int)threadIdx.x + 256 * i;
-            if (UNITS % 256 != 0 && u >= UNITS) break;
+            const int u = c.t + 128 * i;
+            uint16_t *o = lds + row_of(u) * LD + k_of(u);
             if constexpr (AL == ALONG_K) {
-                *reinterpret_cast<uint4 *>(lds + (u / (BK / 8)) * LD + (u % (BK / 8)) * 8) = v[i][0];
+                *reinterpret_cast<uint2 *>(o) = make_uint2(v[i].x, v[i].y);
+                *reinterpret_cast<uint2 *>(o + 4) = make_uint2(v[i].z, v[i].w);
             } else {
-                uint16_t *o = lds + (u % (BR / 8)) * 8 * LD + (u / (BR / 8)) * 4;
+                const uint32_t k0[2] = {v[2 * i].x, v[2 * i].y}, k1[2] = {v[2 * i].z, v[2 * i].w};
+                const uint32_t k2[2] = {v[2 * i + 1].x, v[2 * i + 1].y}, k3[2] = {v[2 * i + 1].z, v[2 * i + 1].w};
 #pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
-                    uint32_t w[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        w[j] = t < 2 ? v[i][j].x : t < 4 ? v[i][j].y : t < 6 ? v[i][j].z : v[i][j].w;
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t sel = (r & 1) ? 0x07060302u : 0x05040100u;
                     uint2 x;
-                    x.x = __builtin_amdgcn_perm(w[1], w[0], sel);
-                    x.y = __builtin_amdgcn_perm(w[3], w[2], sel);
-                    *reinterpret_cast<uint2 *>(o + t * LD) = x;
+                    x.x = __builtin_amdgcn_perm(k1[r >> 1], k0[r >> 1], sel);
+                    x.y = __builtin_amdgcn_perm(k3[r >> 1], k2[r >> 1], sel);
+                    *reinterpret_cast<uint2 *>(o + r * LD) = x;
                 }
             }
         }
@@ -218,16 +259,29 @@ __device__ __forceinline__ void tile_gemm(const TileArgs &g, int bm, int bn, uin
     for (int a = 0; a < TM; ++a)
 #pragma unroll
         for (int b = 0; b < TN; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-    if (g.clear && bm == 0 && bn == 0 && tid < 2) g.clear[tid] = 0.0f;
-    const bool sums = g.rowsum && bn == 0;
+    // one block more per row of blocks adds A's rows and multiplies nothing: the sums are a serial
+    // chain as long as the contraction, which in a multiplying block came on top of its products
+    const bool sums = n0 >= g.N;
     float rs = 0.0f;
-    SA sa[PF];
-    SB sb[PF];
+    // waves 0 and 1 move A, waves 2 and 3 move B
+    const bool first = wave < 2;
+    constexpr bool SAME = AA == AB && BM == BN;
+    constexpr int NP = SA::PER > SB::PER ? SA::PER : SB::PER;
+    Mover<NP> mv;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) mv.ptr[i] = g.A;
+    uint4 v[PF][SA::REGS > SB::REGS ? SA::REGS : SB::REGS];
+    mv.t = tid & 127;
+    if (SAME) SA::init(mv, first ? g.A : g.B, first ? g.lda : g.ldb, first ? m0 : n0, first ? g.M : g.N);
+    else if (first) SA::init(mv, g.A, g.lda, m0, g.M);
+    else SB::init(mv, g.B, g.ldb, n0, g.N);
     const int nk = (g.K + BK - 1) / BK;
-    const auto fetch = [&](int slot, int it) {
+    const auto fetch = [&](int slot, int it) __attribute__((always_inline)) {
         if (it < nk) {
-            sa[slot].load(g.A, g.lda, m0, g.M, it * BK, g.K);
-            sb[slot].load(g.B, g.ldb, n0, g.N, it * BK, g.K);
+            if (SAME || first) SA::load(mv, v[slot], it * BK, g.K);
+            else SB::load(mv, v[slot], it * BK, g.K);
+#pragma unroll
+            for (int i = 0; i < NP; ++i) mv.ptr[i] += mv.step;
         }
     };
 #pragma unroll
@@ -240,12 +294,14 @@ __device__ __forceinline__ void tile_gemm(const TileArgs &g, int bm, int bn, uin
             // two buffers and one barrier per tile: a wave that writes tile it + 1 has passed the barrier
             // of tile it, so every wave is done with the buffer of tile it - 1
             uint16_t *As = lds + (it & 1) * BUF, *Bs = As + BM * LD;
-            sa[p].store(As);
-            sb[p].store(Bs);
+            if (SAME) SA::store(mv, v[p], first ? As : Bs);
+            else if (first) SA::store(mv, v[p], As);
+            else SB::store(mv, v[p], Bs);
             __syncthreads();
             fetch(p, it + PF);
 #pragma unroll
             for (int kk = 0; kk < BK; kk += 16) {
+                if (sums) break;
                 v4s a[TM], b[TN];
 #pragma unroll
                 for (int mi = 0; mi < TM; ++mi)
@@ -261,11 +317,11 @@ __device__ __forceinline__ void tile_gemm(const TileArgs &g, int bm, int bn, uin
             }
             if (sums && tid < BM) {
 #pragma unroll
-                for (int k = 0; k < BK; k += 8) {
-                    const uint4 x = *reinterpret_cast<const uint4 *>(As + tid * LD + k);
-                    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+                for (int k = 0; k < BK; k += 4) {
+                    const uint2 x = *reinterpret_cast<const uint2 *>(As + tid * LD + k);
+                    const uint32_t w[2] = {x.x, x.y};
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) {
+                    for (int t = 0; t < 2; ++t) {
                         rs += __uint_as_float(w[t] << 16);
                         rs += __uint_as_float(w[t] & 0xffff0000u);
                     }
@@ -273,7 +329,10 @@ __device__ __forceinline__ void tile_gemm(const TileArgs &g, int bm, int bn, uin
             }
         }
     }
-    if (sums && tid < BM && m0 + tid < g.M) g.rowsum[m0 + tid] = rs;
+    if (sums) {
+        if (tid < BM && m0 + tid < g.M) g.rowsum[m0 + tid] = rs;
+        return;
+    }
 #pragma unroll
     for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
@@ -295,7 +354,7 @@ __device__ __forceinline__ void tile_gemm(const TileArgs &g, int bm, int bn, uin
 
 template <int BM, int BN, int BK, Along AA, Along AB, int PF>
 __global__ __launch_bounds__(256) void tile_kernel(TileArgs g) {
-    __shared__ __align__(16) uint16_t lds[2 * (BM + BN) * (BK + 8)];
+    __shared__ __align__(16) uint16_t lds[2 * (BM + BN) * (BK + 4)];
     tile_gemm<BM, BN, BK, AA, AB, PF>(g, blockIdx.y, blockIdx.x, lds);
 }
 
@@ -304,7 +363,7 @@ __global__ __launch_bounds__(256) void tile_kernel(TileArgs g) {
 // across it).  Neither fills the device alone.
 template <int BM1, int BN1, int BK1, int PF1, int BM2, int BN2, int BK2, int PF2>
 __global__ __launch_bounds__(256) void tile_pair_kernel(TileArgs g1, int nb1, int nn1, TileArgs g2, int nn2) {
-    constexpr int L1 = 2 * (BM1 + BN1) * (BK1 + 8), L2 = 2 * (BM2 + BN2) * (BK2 + 8);
+    constexpr int L1 = 2 * (BM1 + BN1) * (BK1 + 4), L2 = 2 * (BM2 + BN2) * (BK2 + 4);
     __shared__ __align__(16) uint16_t lds[L1 > L2 ? L1 : L2];
     const int b = blockIdx.x;
     if (b < nb1)
@@ -314,10 +373,12 @@ __global__ __launch_bounds__(256) void tile_pair_kernel(TileArgs g1, int nb1, in
 }
 
 static int tiles(int n, int b) { return (n + b - 1) / b; }
+// blocks along n: the products' and, with row sums, one for those
+static int tiles_n(const TileArgs &g, int b) { return tiles(g.N, b) + (g.rowsum ? 1 : 0); }
 
 template <int BM, int BN, int BK, Along AA, Along AB, int PF>
 static int tile_launch(const TileArgs &g, hipStream_t st) {
-    hipLaunchKernelGGL((tile_kernel<BM, BN, BK, AA, AB, PF>), dim3(tiles(g.N, BN), tiles(g.M, BM)), dim3(256), 0, st, g);
+    hipLaunchKernelGGL((tile_kernel<BM, BN, BK, AA, AB, PF>), dim3(tiles_n(g, BN), tiles(g.M, BM)), dim3(256), 0, st, g);
     MHIP(hipGetLastError());
     return 0;
 }
@@ -334,24 +395,32 @@ extern "C" int song_gemm_bf16(int M, int N, int K, const uint16_t *d_a, int sam,
 // ---------------------------------------------------------------- loss, sums, Adam
 
 // One block of four waves per row: softmax cross-entropy over the first C logits against the label,
-// squared error of logit C against the stop target; writes dZ (bf16) and adds the batch means of both
-// losses to loss[0..1].  Every exponential is computed once, by all waves, and kept in LDS (C + 1
+// squared error of logit C against the stop target; writes dZ (bf16) and the row's share of the batch
+// means of both losses.  Every exponential is computed once, by all waves, and kept in LDS (C + 1
 // floats); the first wave adds them, lane l the columns l, l + 64, ... in ascending order and then
 // the lanes in halving steps, the order a single wave per row has, so the sum does not depend on the
 // waves.  Rows too wide for LDS (IN_LDS false) compute the exponentials again where they are used.
-// One wave per row that computed each exponential twice took 64 us for 1,024 rows of 4,097.
+// One wave per row that computed each exponential twice took 64 us for 1,024 rows of 4,097; four waves
+// that added the losses to one pair of floats took 39 us, most of it those 2,048 atomics; now 10 us.
 constexpr int LOSS_LDS_CLASSES = 12288;  // 48 KB: three blocks fit a CU's LDS
 template <bool IN_LDS>
 __global__ __launch_bounds__(256) void loss_kernel(const float *Z, int ldz, int C, const int *labels, const float *stop_t,
-                                                   int B, float stop_w, uint16_t *dZ, int lddz, float *loss) {
+                                                   int B, float stop_w, uint16_t *dZ, int lddz, float2 *row_loss) {
     extern __shared__ __align__(16) float ex[];
     __shared__ float red[8];
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float *z = Z + (long long)row * ldz;
+    uint16_t *dz = dZ + (long long)row * lddz;
+    const int C4 = C & ~3;  // columns taken four at a time (rows are 16-byte aligned), then the rest
     float mx = -INFINITY;
-    for (int c = tid; c < C; c += 256) {
-        const float v = z[c];
-        if (IN_LDS) ex[c] = v;
+    for (int c = 4 * tid; c < C4; c += 1024) {
+        const float4 v = *reinterpret_cast<const float4 *>(z + c);
+        if (IN_LDS) *reinterpret_cast<float4 *>(ex + c) = v;
+        mx = fmaxf(fmaxf(fmaxf(mx, v.x), fmaxf(v.y, v.z)), v.w);
+    }
+    if (C4 + tid < C) {
+        const float v = z[C4 + tid];
+        if (IN_LDS) ex[C4 + tid] = v;
         mx = fmaxf(mx, v);
     }
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
@@ -364,7 +433,16 @@ __global__ __launch_bounds__(256) void loss_kernel(const float *Z, int ldz, int 
     }
     if (wave == 0) {
         float se = 0.0f;
-        for (int c = lane; c < C; c += 64) se += IN_LDS ? ex[c] : expf(z[c] - mx);
+        int c = lane;
+        if (IN_LDS)
+            for (; c + 7 * 64 < C; c += 512) {  // eight reads in flight, added in order
+                float e[8];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) e[t] = ex[c + 64 * t];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) se += e[t];
+            }
+        for (; c < C; c += 64) se += IN_LDS ? ex[c] : expf(z[c] - mx);
         for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o);
         if (lane == 0) red[4] = se;
     }
@@ -372,15 +450,41 @@ __global__ __launch_bounds__(256) void loss_kernel(const float *Z, int ldz, int 
     const float se = red[4];
     const int lab = labels[row];
     const float inv = 1.0f / (float)B;
-    for (int c = tid; c < C; c += 256) {
-        const float p = (IN_LDS ? ex[c] : expf(z[c] - mx)) / se;
-        dZ[(long long)row * lddz + c] = f2bf((p - (c == lab ? 1.0f : 0.0f)) * inv);
+    const auto grad = [&](float e, int c) { return f2bf((e / se - (c == lab ? 1.0f : 0.0f)) * inv); };
+    for (int c = 4 * tid; c < C4; c += 1024) {
+        float4 e = *reinterpret_cast<const float4 *>(IN_LDS ? ex + c : z + c);
+        if (!IN_LDS) e = make_float4(expf(e.x - mx), expf(e.y - mx), expf(e.z - mx), expf(e.w - mx));
+        *reinterpret_cast<ushort4 *>(dz + c) = make_ushort4(grad(e.x, c), grad(e.y, c + 1), grad(e.z, c + 2), grad(e.w, c + 3));
+    }
+    if (C4 + tid < C) {
+        const int c = C4 + tid;
+        dz[c] = grad(IN_LDS ? ex[c] : expf(z[c] - mx), c);
     }
     if (tid == 0) {
         const float diff = z[C] - stop_t[row];
-        dZ[(long long)row * lddz + C] = f2bf(2.0f * stop_w * diff * inv);
-        atomicAdd(&loss[0], (logf(se) + mx - z[lab]) * inv);
-        atomicAdd(&loss[1], diff * diff * inv);
+        dz[C] = f2bf(2.0f * stop_w * diff * inv);
+        row_loss[row] = make_float2((logf(se) + mx - z[lab]) * inv, diff * diff * inv);
+    }
+}
+
+// the batch's losses from its rows', when they are asked for
+__global__ __launch_bounds__(256) void loss_sum_kernel(const float2 *row_loss, int B, float *loss) {
+    __shared__ float2 part[4];
+    const int tid = threadIdx.x;
+    float2 s = make_float2(0.0f, 0.0f);
+    for (int i = tid; i < B; i += 256) {
+        s.x += row_loss[i].x;
+        s.y += row_loss[i].y;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        s.x += __shfl_xor(s.x, o);
+        s.y += __shfl_xor(s.y, o);
+    }
+    if ((tid & 63) == 0) part[tid >> 6] = s;
+    __syncthreads();
+    if (tid == 0) {
+        loss[0] = (part[0].x + part[1].x) + (part[2].x + part[3].x);
+        loss[1] = (part[0].y + part[1].y) + (part[2].y + part[3].y);
     }
 }
 
@@ -827,6 +931,7 @@ struct song_mlp {
     int ldz = 0;              // row stride of Z and dZ: C + 1 rounded up to 8 (16-byte rows)
     uint16_t *H1 = nullptr, *H2 = nullptr, *dZ = nullptr, *dH2 = nullptr, *dH1 = nullptr;
     float *Z = nullptr, *loss = nullptr;
+    float2 *row_loss = nullptr;  // each row's share of the two losses
     uint16_t *Xa = nullptr;  // aligned copy of inputs that are not
     int t = 0;
 };
@@ -906,7 +1011,8 @@ extern "C" int song_mlp_create(int in_dim, int hidden, int n_classes, int max_ba
     const long long B = max_batch, LZ = m->ldz;
     if (hipMalloc(&m->H1, B * hidden * 2) || hipMalloc(&m->H2, B * hidden * 2) || hipMalloc(&m->dZ, B * LZ * 2) ||
         hipMalloc(&m->dH2, B * hidden * 2) || hipMalloc(&m->dH1, B * hidden * 2) || hipMalloc(&m->Z, B * LZ * 4) ||
-        hipMalloc(&m->loss, 8) || hipMalloc(&m->Xa, B * m->width * 2))
+        hipMalloc(&m->loss, 8) || hipMalloc(&m->Xa, B * m->width * 2) ||
+        hipMalloc(&m->row_loss, B * sizeof(float2)))
         return bad("activations");
     if (hipMemcpy(m->P, init.data(), o * 4, hipMemcpyHostToDevice) || hipMemset(m->Mo, 0, o * 4) ||
         hipMemset(m->Vo, 0, o * 4) || hipMemset(m->G, 0, o * 4)) {
@@ -924,7 +1030,7 @@ extern "C" int song_mlp_create(int in_dim, int hidden, int n_classes, int max_ba
 extern "C" int song_mlp_destroy(song_mlp *m) {
     if (!m) return 0;
     void *ptrs[] = {m->P, m->G, m->Mo, m->Vo, m->Wb[0], m->Wb[1], m->Wb[2], m->W3i, m->H1, m->H2, m->dZ, m->dH2,
-                    m->dH1, m->Z, m->loss, m->Xa};
+                    m->dH1, m->Z, m->loss, m->row_loss, m->Xa};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     delete m;
@@ -983,7 +1089,6 @@ extern "C" int song_mlp_loss_grad(song_mlp *m, const uint16_t *d_x, const int *d
     g.ldcb = Hd;
     g.bias = b1;
     g.relu = 1;
-    g.clear = m->loss;
     if (tile_launch<32, 32, 64, ALONG_K, ALONG_K, 2>(g, st)) return -2;
     g = args(batch, Hd, Hd, m->H1, Hd, m->Wb[1], Hd);
     g.Cb = m->H2;
@@ -995,11 +1100,11 @@ extern "C" int song_mlp_loss_grad(song_mlp *m, const uint16_t *d_x, const int *d
     g.C = m->Z;
     g.ldc = LZ;
     g.bias = b3;
-    if (tile_launch<64, 64, 64, ALONG_K, ALONG_K, 2>(g, st)) return -2;
+    if (tile_launch<64, 64, 32, ALONG_K, ALONG_K, 2>(g, st)) return -2;
     const bool in_lds = m->C <= LOSS_LDS_CLASSES;
     hipLaunchKernelGGL(in_lds ? loss_kernel<true> : loss_kernel<false>, dim3(batch), dim3(256),
                        in_lds ? (size_t)m->C * sizeof(float) : 0, st, m->Z, LZ, m->C, d_labels, d_stop, batch,
-                       stop_weight, m->dZ, LZ, m->loss);
+                       stop_weight, m->dZ, LZ, m->row_loss);
     MHIP(hipGetLastError());
     // backward: dH2 = dZ W3 * (H2 > 0) beside dW3 = dZ^T H2 and db3, then dH1 beside dW2 and db2, then dW1
     TileArgs gi = args(batch, Hd, NO, m->dZ, LZ, m->Wb[2], Hd);
@@ -1012,9 +1117,9 @@ extern "C" int song_mlp_loss_grad(song_mlp *m, const uint16_t *d_x, const int *d
     gw.ldc = Hd;
     gw.rowsum = G + m->off[5];
     {
-        const int nb1 = tiles(batch, 32) * tiles(Hd, 32), nb2 = tiles(NO, 64) * tiles(Hd, 64);
+        const int nb1 = tiles(batch, 32) * tiles(Hd, 32), nb2 = tiles(NO, 64) * tiles_n(gw, 64);
         hipLaunchKernelGGL((tile_pair_kernel<32, 32, 128, 2, 64, 64, 32, 2>), dim3(nb1 + nb2), dim3(256), 0, st, gi, nb1,
-                           tiles(Hd, 32), gw, tiles(Hd, 64));
+                           tiles(Hd, 32), gw, tiles_n(gw, 64));
         MHIP(hipGetLastError());
     }
     gi = args(batch, Hd, Hd, m->dH2, Hd, m->Wb[1], Hd);
@@ -1027,17 +1132,19 @@ extern "C" int song_mlp_loss_grad(song_mlp *m, const uint16_t *d_x, const int *d
     gw.ldc = Hd;
     gw.rowsum = G + m->off[3];
     {
-        const int nb1 = tiles(batch, 32) * tiles(Hd, 32), nb2 = tiles(Hd, 32) * tiles(Hd, 32);
-        hipLaunchKernelGGL((tile_pair_kernel<32, 32, 64, 2, 32, 32, 64, 2>), dim3(nb1 + nb2), dim3(256), 0, st, gi, nb1,
-                           tiles(Hd, 32), gw, tiles(Hd, 32));
+        const int nb1 = tiles(batch, 32) * tiles(Hd, 32), nb2 = tiles(Hd, 32) * tiles_n(gw, 32);
+        hipLaunchKernelGGL((tile_pair_kernel<32, 32, 128, 2, 32, 32, 128, 2>), dim3(nb1 + nb2), dim3(256), 0, st, gi, nb1,
+                           tiles(Hd, 32), gw, tiles_n(gw, 32));
         MHIP(hipGetLastError());
     }
     g = args(Hd, W, batch, m->dH1, Hd, x, W);
     g.C = G + m->off[0];
     g.ldc = W;
     g.rowsum = G + m->off[1];
-    if (tile_launch<32, 32, 64, ALONG_ROW, ALONG_ROW, 2>(g, st)) return -2;
+    if (tile_launch<32, 32, 128, ALONG_ROW, ALONG_ROW, 2>(g, st)) return -2;
     if (loss_out) {
+        hipLaunchKernelGGL(loss_sum_kernel, dim3(1), dim3(256), 0, st, m->row_loss, batch, m->loss);
+        MHIP(hipGetLastError());
         MHIP(hipMemcpyAsync(loss_out, m->loss, 8, hipMemcpyDeviceToHost, st));
         MHIP(hipStreamSynchronize(st));
     }
