@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -510,11 +511,12 @@ __device__ __forceinline__ void adam_one(const AdamArgs &a, float gi, float &p, 
 }
 
 // Every parameter once: with ADAM the update, then the bf16 copies of the weights, the output
-// weights twice -- row by row for the products, and for inference in k quads: fragment (k-step s,
-// k-quad q, column n) = W3[n][16s + 4q .. +4) at W3i[((4s + q) * npad + n) * 4], zero for n >= rows3,
-// so that the 16 columns a lane group reads per step are one aligned 128-byte run.  The first blocks
+// weights twice -- row by row for the products, and for inference in pairs of k quads: W3[n][32s + 4q
+// .. +4) and W3[n][32s + 16 + 4q .. +4) at W3i[((4s + q) * npad + n) * 8], zero for n >= rows3 and past
+// the last hidden unit, so that a lane reads its fragments of two k-steps in one 16-byte load and the
+// 16 columns of a lane group are one aligned 256-byte run.  The first blocks
 // take W3 in tiles of 16 rows x 64 columns, four columns per lane (64-byte runs of the float arrays,
-// 128-byte runs of W3i); the rest take the other segments in order.  Bound by memory: 30 bytes per
+// half-filled 256-byte runs of W3i); the rest take the other segments in order.  Bound by memory: 30 bytes per
 // parameter.  As five kernels (update, three conversions, interleave) a step took 26 us at 1.16
 // million parameters and read the new weights three times.
 template <bool ADAM>
@@ -542,7 +544,8 @@ __global__ __launch_bounds__(256) void refresh_kernel(AdamArgs a, ParamCopies c,
             h[0] = f2bf(p.x), h[1] = f2bf(p.y), h[2] = f2bf(p.z), h[3] = f2bf(p.w);
             *reinterpret_cast<ushort4 *>(c.Wb[2] + (long long)n * c.hidden + k) = make_ushort4(h[0], h[1], h[2], h[3]);
         }
-        *reinterpret_cast<ushort4 *>(c.W3i + ((long long)(k >> 2) * c.npad + n) * 4) = make_ushort4(h[0], h[1], h[2], h[3]);
+        const long long sq = (long long)(k >> 5) * 4 + ((k >> 2) & 3);
+        *reinterpret_cast<ushort4 *>(c.W3i + (sq * c.npad + n) * 8 + ((k >> 4) & 1) * 4) = make_ushort4(h[0], h[1], h[2], h[3]);
         return;
     }
     // W1 b1 W2 b2 are one run, b3 is the last
@@ -612,146 +615,73 @@ __global__ __launch_bounds__(64) void features_kernel(const float *Q, int dim, c
 
 // ---------------------------------------------------------------- fused inference
 
-// queries per workgroup: 16 rows (MI = 1 row tile) -- a 10k-query batch launches 625 workgroups,
-// two or three per CU, and each wave's chain of MFMAs and softmax updates is half that of 32 rows;
-// the output weights are read twice as often, from L2.  For 10k queries: 16 rows 197 us, 32 rows
-// 256 us, 64 rows 447 us (157 workgroups, one wave per SIMD)
-constexpr int IQ = 16;
-constexpr int MI = IQ / 16;
-// waves per workgroup: they split the output layer's columns (64 per wave and chunk) and the
-// hidden units (slices of 64); with 16 rows, 2 waves per group measured 319 us and 8 waves 206 us
-constexpr int IW = 4;
-constexpr int IT = 64 * IW;  // threads per workgroup
-
 struct InferArgs {
     const uint16_t *X;
     int batch, width, hidden, C;
     const uint16_t *W1, *W2, *W3;
-    const uint16_t *W3i;  // W3 in the k-quad interleaved layout, npad columns
+    const uint16_t *W3i;  // W3 in the layout of refresh_kernel, npad columns
     int npad;
     const float *b1, *b2, *b3;
     int *top2;  // batch x 2 pivot indices (best first)
     float *conf, *stop, *logits;
     const int *nbr;  // C x n_nbr pivot neighbourhoods (row a starts with a) or null
     int n_nbr;
+    int x16;  // 1: X can be read in 16-byte units
 };
 
-// One dense layer on the LDS tile: accumulators of in[IQ rows] . W[n]^T for the 64-column
-// slice [n0, n0+64) of this wave (MI x 4 MFMA tiles).  K is a multiple of 16, so every
-// fragment (4 consecutive k of one row or column) is one aligned 8-byte load; the next
-// k-step's weight fragments are loaded while the current step's MFMAs run (a deeper ring of
-// in-flight weight loads measured no faster).
-__device__ __forceinline__ void tile_layer(const uint16_t *in, int ldin, int K, const uint16_t *W, int N, int n0,
-                                           v4f (&acc)[MI][4]) {
-    const int lane = threadIdx.x & 63;
-    const int kq = 4 * (lane >> 4);
-#pragma unroll
-    for (int a = 0; a < MI; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-    const uint16_t *wrow[4];
-    bool ok[4];
-    v4s bf[4];
-#pragma unroll
-    for (int ni = 0; ni < 4; ++ni) {
-        const int n = n0 + ni * 16 + (lane & 15);
-        ok[ni] = n < N;
-        wrow[ni] = W + (long long)(ok[ni] ? n : 0) * K + kq;
-        bf[ni] = ok[ni] ? *reinterpret_cast<const v4s *>(wrow[ni]) : v4s{0, 0, 0, 0};
-    }
+// exp(x) for finite x <= REF_SPAN to within an ulp or two: 2^(x log2 e) by the hardware's exponential, the
+// product's rounding error carried along and put back as a first-order factor
+__device__ __forceinline__ float exp_mid(float x) {
+    const float L = 1.44269502f, Ll = 1.92596303e-8f, ln2 = 0.693147182f;  // L + Ll = log2 e
+    const float hi = x * L;
+    const float lo = fmaf(x, Ll, fmaf(x, L, -hi));
+    const float e = __builtin_amdgcn_exp2f(hi);
+    return fmaf(e, lo * ln2, e);
+}
+
+// One hidden layer on the LDS tile: out[r][n] = relu(in[r] . W[n] + bias[n]) for this block's rows,
+// the waves taking 16 columns at a time.  The weight fragments of eight k-steps are loaded together,
+// so a tile waits for memory once or twice, not once per step.
+template <int MI, int WAVES>
+__device__ __forceinline__ void hidden_layer(const uint16_t *in, int ldin, int K, const uint16_t *W, const float *bias,
+                                             int N, uint16_t *out, int ldo) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kq = 4 * (lane >> 4);
     const uint16_t *arow = in + (lane & 15) * ldin + kq;
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        const bool more = k0 + 16 < K;
-        v4s nb[4];
+    for (int n0 = wave * 16; n0 < N; n0 += WAVES * 16) {  // (N is a multiple of 16)
+        const int n = n0 + (lane & 15);
+        const uint16_t *w = W + (size_t)n * K + kq;
+        v4f acc[MI];
 #pragma unroll
-        for (int ni = 0; ni < 4; ++ni)
-            nb[ni] = (ok[ni] && more) ? *reinterpret_cast<const v4s *>(wrow[ni] + k0 + 16) : v4s{0, 0, 0, 0};
+        for (int mi = 0; mi < MI; ++mi) acc[mi] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int k0 = 0; k0 < K; k0 += 128) {
+            v4s b[8];
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi) {
-            const v4s af = *reinterpret_cast<const v4s *>(arow + mi * 16 * ldin + k0);
+            for (int t = 0; t < 8; ++t) b[t] = *reinterpret_cast<const v4s *>(w + min(k0 + 16 * t, K - 16));
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni)
-                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af, bf[ni], acc[mi][ni], 0, 0, 0);
+            for (int t = 0; t < 8; ++t) {
+                if (k0 + 16 * t >= K) break;
+#pragma unroll
+                for (int mi = 0; mi < MI; ++mi)
+                    acc[mi] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                        *reinterpret_cast<const v4s *>(arow + mi * 16 * ldin + k0 + 16 * t), b[t], acc[mi], 0, 0, 0);
+            }
         }
+        const float bn = bias[n];
 #pragma unroll
-        for (int ni = 0; ni < 4; ++ni) bf[ni] = nb[ni];
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                out[(mi * 16 + 4 * (lane >> 4) + t) * ldo + n] = f2bf(fmaxf(acc[mi][t] + bn, 0.0f));
     }
 }
 
-// As tile_layer, with the weights in the k-quad interleaved layout (refresh_kernel): a lane
-// group's 16 fragments of one step are one contiguous 128-byte run (four full cache lines per
-// load instead of 32 bytes of sixteen).  The lanes take the same k as in tile_layer, so the
-// accumulators are identical.
-__device__ __forceinline__ void tile_layer_il(const uint16_t *in, int ldin, int K, const uint16_t *Wi, int N, int npad,
-                                              int n0, v4f (&acc)[MI][4]) {
-    const int lane = threadIdx.x & 63;
-    const int q = lane >> 4, kq = 4 * q;
-#pragma unroll
-    for (int a = 0; a < MI; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = v4f{0.f, 0.f, 0.f, 0.f};
-    const long long sstride = 16LL * npad;  // elements per k-step: 4 quads x npad columns x 4
-    const uint16_t *wb[4];
-    bool ok[4];
-    v4s bf[4];
-#pragma unroll
-    for (int ni = 0; ni < 4; ++ni) {
-        const int n = n0 + ni * 16 + (lane & 15);
-        ok[ni] = n < N;
-        wb[ni] = Wi + ((long long)q * npad + (ok[ni] ? n : 0)) * 4;
-        bf[ni] = ok[ni] ? *reinterpret_cast<const v4s *>(wb[ni]) : v4s{0, 0, 0, 0};
-    }
-    const uint16_t *arow = in + (lane & 15) * ldin + kq;
-    for (int k0 = 0, st = 0; k0 < K; k0 += 16, ++st) {
-        const bool more = k0 + 16 < K;
-        v4s nb[4];
-#pragma unroll
-        for (int ni = 0; ni < 4; ++ni)
-            nb[ni] = (ok[ni] && more) ? *reinterpret_cast<const v4s *>(wb[ni] + (st + 1) * sstride) : v4s{0, 0, 0, 0};
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi) {
-            const v4s af = *reinterpret_cast<const v4s *>(arow + mi * 16 * ldin + k0);
-#pragma unroll
-            for (int ni = 0; ni < 4; ++ni)
-                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af, bf[ni], acc[mi][ni], 0, 0, 0);
-        }
-#pragma unroll
-        for (int ni = 0; ni < 4; ++ni) bf[ni] = nb[ni];
-    }
-}
-
-// running softmax state of a row: top two (value, index) and the sum of exp(v - v1)
+// softmax state of a row: top two (value, index) and the sum of exp(v - v1)
 struct Soft {
     float v1, v2, s;
     int a1, a2;
 };
 __device__ __forceinline__ bool better(float v, int a, float w, int b) { return v > w || (v == w && a < b); }
 __device__ __forceinline__ Soft soft_empty() { return Soft{-INFINITY, -INFINITY, 0.0f, 0x7fffffff, 0x7fffffff}; }
-// the (value, index) pair into the top two, without branches
-__device__ __forceinline__ void top2_add(Soft &t, float v, int a) {
-    const bool b1 = better(v, a, t.v1, t.a1), b2 = better(v, a, t.v2, t.a2);
-    const float nv2 = b1 ? t.v1 : (b2 ? v : t.v2);
-    const int na2 = b1 ? t.a1 : (b2 ? a : t.a2);
-    t.v1 = b1 ? v : t.v1;
-    t.a1 = b1 ? a : t.a1;
-    t.v2 = nv2;
-    t.a2 = na2;
-}
-// four values of one row at once (-inf where absent): one rescale of the running sum to the new
-// maximum, four exponentials, then the top two
-__device__ __forceinline__ void soft_add4(Soft &t, const float (&v)[4], const int (&a)[4]) {
-    const float m = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
-    if (m == -INFINITY) return;
-    const float ref = fmaxf(m, t.v1);
-    float s = t.v1 == -INFINITY ? 0.0f : t.s * expf(t.v1 - ref);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s += expf(v[i] - ref);  // exp(-inf) = 0
-    t.s = s;
-    // the sum is kept relative to the top value: ref becomes v1 below whenever m > v1
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (v[i] != -INFINITY) top2_add(t, v[i], a[i]);
-}
 __device__ __forceinline__ Soft soft_merge(const Soft &x, const Soft &y) {
     if (y.v1 == -INFINITY) return x;
     if (x.v1 == -INFINITY) return y;
@@ -783,87 +713,177 @@ __device__ __forceinline__ Soft soft_merge(const Soft &x, const Soft &y) {
     return t;
 }
 
-__global__ __launch_bounds__(IT) void infer_kernel(InferArgs a) {
+// A row's running state over the columns one lane owns, in ascending order: the top two, and the sum
+// of exp(v - ref) for a reference that only moves when a value exceeds it by REF_SPAN (the sum of at
+// most 2^31 terms below e^REF_SPAN stays finite), so that a value costs one exponential.
+constexpr float REF_SPAN = 40.0f;
+struct Lane {
+    float v1, v2, s, ref;
+    int a1, a2;
+};
+// `v` of column `a`, larger than every column before it (a tie keeps the earlier one), into the top two
+__device__ __forceinline__ void lane_top(Lane &t, float v, int a) {
+    const bool b1 = v > t.v1, b2 = v > t.v2;
+    t.a2 = b1 ? t.a1 : (b2 ? a : t.a2);
+    t.a1 = b1 ? a : t.a1;
+    t.v2 = b1 ? t.v1 : (b2 ? v : t.v2);
+    t.v1 = b1 ? v : t.v1;
+}
+// one value into the sum, whatever it is (NaN stays NaN, -inf adds nothing)
+__device__ __forceinline__ void lane_sum(Lane &t, float v) {
+    if (v - t.ref > REF_SPAN) {
+        t.s *= expf(t.ref - v);
+        t.ref = v;
+    }
+    t.s += expf(v - t.ref);
+}
+
+// Fused inference of 16 MI queries per block by WAVES waves: two hidden layers, the output layer with a
+// running softmax, the confidence.  In the output layer a wave takes 64 columns at a time (4 column
+// tiles x MI row tiles of accumulators); its weights come from W3i 16 bytes per lane, two k-steps per
+// load, one step ahead across the column groups, so the softmax of a group covers the first loads of
+// the next.  Bound: the vector instructions of the softmax (about 17 per logit) and the L2 reads of the
+// weights (each block reads all of them), 136-256-256-4,097: 10,000 queries 213 -> 101 us, 33 queries
+// 197 -> 47 us against four waves per 16 rows with two bytes of X, eight of W per load and five
+// library exponentials per four logits.
+template <int MI, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void infer_kernel(InferArgs a) {
+    constexpr int IQ = 16 * MI, IT = 64 * WAVES;
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r0 = blockIdx.x * IQ;
-    const int ldx = a.width + 8, ldh = a.hidden + 8;
-    uint16_t *X = reinterpret_cast<uint16_t *>(smem);
+    const int kp = (a.hidden + 31) & ~31;  // contraction of the output layer, padded with zeros
+    const int ldx = a.width + 8, ldh = kp + 8;
+    uint16_t *H2 = reinterpret_cast<uint16_t *>(smem);
+    float *stp = reinterpret_cast<float *>(H2 + IQ * ldh);  // [IQ]
+    uint16_t *X = reinterpret_cast<uint16_t *>(stp + IQ);
     uint16_t *H1 = X + IQ * ldx;
-    uint16_t *H2 = H1 + IQ * ldh;
-    Soft *part = reinterpret_cast<Soft *>(H2 + IQ * ldh);  // [IW waves][IQ]
-    Soft *run = part + IW * IQ;                             // [IQ]
-    float *stp = reinterpret_cast<float *>(run + IQ);       // [IQ]
+    // once the hidden layers are done, in their place:
+    Soft *part = reinterpret_cast<Soft *>(X);  // [WAVES][IQ]
+    Soft *run = part + WAVES * IQ;             // [IQ]
 
-    for (int e = tid; e < IQ * a.width; e += IT) {
-        const int r = e / a.width, c = e % a.width;
-        X[r * ldx + c] = (r0 + r < a.batch) ? a.X[(long long)(r0 + r) * a.width + c] : (uint16_t)0;
+    if (a.x16) {
+        const int u = a.width / 8;
+        for (int e = tid; e < IQ * u; e += IT) {
+            const int r = e / u, c = (e % u) * 8;
+            *reinterpret_cast<uint4 *>(X + r * ldx + c) =
+                r0 + r < a.batch ? *reinterpret_cast<const uint4 *>(a.X + (size_t)(r0 + r) * a.width + c)
+                                 : make_uint4(0u, 0u, 0u, 0u);
+        }
+    } else {
+        for (int e = tid; e < IQ * a.width; e += IT) {
+            const int r = e / a.width, c = e % a.width;
+            X[r * ldx + c] = (r0 + r < a.batch) ? a.X[(size_t)(r0 + r) * a.width + c] : (uint16_t)0;
+        }
     }
-    for (int r = tid; r < IQ; r += IT) run[r] = soft_empty();
+    if (kp > a.hidden)
+        for (int e = tid; e < IQ * 16; e += IT) H2[(e >> 4) * ldh + a.hidden + (e & 15)] = 0;
+    __syncthreads();
+    hidden_layer<MI, WAVES>(X, ldx, a.width, a.W1, a.b1, a.hidden, H1, ldh);
+    __syncthreads();
+    hidden_layer<MI, WAVES>(H1, ldh, a.hidden, a.W2, a.b2, a.hidden, H2, ldh);
     __syncthreads();
 
-    v4f acc[MI][4];
-    // hidden layers: the waves split the hidden units in slices of 64
-    for (int layer = 0; layer < 2; ++layer) {
-        const uint16_t *in = layer == 0 ? X : H1;
-        const int ldin = layer == 0 ? ldx : ldh, K = layer == 0 ? a.width : a.hidden;
-        const uint16_t *W = layer == 0 ? a.W1 : a.W2;
-        const float *bias = layer == 0 ? a.b1 : a.b2;
-        uint16_t *out = layer == 0 ? H1 : H2;
-        for (int n0 = wave * 64; n0 < a.hidden; n0 += IT) {
-            tile_layer(in, ldin, K, W, a.hidden, n0, acc);
-#pragma unroll
-            for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-                for (int ni = 0; ni < 4; ++ni)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int r = mi * 16 + 4 * (lane >> 4) + j, n = n0 + ni * 16 + (lane & 15);
-                        if (n < a.hidden) out[r * ldh + n] = f2bf(fmaxf(acc[mi][ni][j] + bias[n], 0.0f));
-                    }
-        }
-        __syncthreads();
-    }
-
-    // output layer in chunks of 64 columns per wave: each lane keeps a running softmax state (top
-    // two and the sum) for each of its rows over the columns it owns; the 16 lanes of a row and
-    // the waves combine once at the end
-    const int NO = a.C + 1;
-    Soft ts[MI][4];
+    const int NO = a.C + 1, S = kp / 32, q = lane >> 4;
+    const int groups = (NO + 63) / 64;
+    Lane ts[MI][4];
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) ts[mi][j] = soft_empty();
-    for (int c0 = 0; c0 < NO; c0 += IT) {
-        const int n0 = c0 + wave * 64;
-        tile_layer_il(H2, ldh, a.hidden, a.W3i, NO, a.npad, n0, acc);
+        for (int j = 0; j < 4; ++j) ts[mi][j] = Lane{-INFINITY, -INFINITY, 0.0f, -FLT_MAX, 0x7fffffff, 0x7fffffff};
+    const uint16_t *arow = H2 + (lane & 15) * ldh + 4 * q;
+    const size_t sstep = (size_t)32 * a.npad;  // elements of W3i per two k-steps
+    const uint16_t *wp = a.W3i + ((size_t)q * a.npad + wave * 64 + (lane & 15)) * 8;
+    uint4 b[4];
+    if (wave < groups) {
+#pragma unroll
+        for (int ni = 0; ni < 4; ++ni) b[ni] = *reinterpret_cast<const uint4 *>(wp + ni * 128);
+    }
+    for (int g = wave; g < groups; g += WAVES) {
+        v4f acc[MI][4];
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = v4f{0.f, 0.f, 0.f, 0.f};
+        float bias[4];
+#pragma unroll
+        for (int ni = 0; ni < 4; ++ni) bias[ni] = a.b3[min(g * 64 + ni * 16 + (lane & 15), NO - 1)];
+        const int tiles_n = min(4, (NO - g * 64 + 15) / 16);  // the last group may hold fewer columns
+        for (int st = 0; st < S; ++st) {
+            // the next two k-steps' weights, or the next group's first (the last group reads its own again)
+            const uint16_t *np = st + 1 < S ? wp + (size_t)(st + 1) * sstep : g + WAVES < groups ? wp + (size_t)WAVES * 512 : wp;
+            uint4 nb[4];
+#pragma unroll
+            for (int ni = 0; ni < 4; ++ni) nb[ni] = *reinterpret_cast<const uint4 *>(np + ni * 128);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                v4s af[MI];
+#pragma unroll
+                for (int mi = 0; mi < MI; ++mi)
+                    af[mi] = *reinterpret_cast<const v4s *>(arow + mi * 16 * ldh + st * 32 + h * 16);
+#pragma unroll
+                for (int ni = 0; ni < 4; ++ni) {
+                    if (ni > 0 && ni >= tiles_n) break;
+                    const uint2 w = h == 0 ? make_uint2(b[ni].x, b[ni].y) : make_uint2(b[ni].z, b[ni].w);
+#pragma unroll
+                    for (int mi = 0; mi < MI; ++mi)
+                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af[mi], __builtin_bit_cast(v4s, w),
+                                                                                acc[mi][ni], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int ni = 0; ni < 4; ++ni) b[ni] = nb[ni];
+        }
+        wp += (size_t)WAVES * 512;
+        const bool whole = g * 64 + 64 <= a.C;  // every column of the group is a pivot's
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int r = mi * 16 + 4 * (lane >> 4) + j;
-                float vv[4];
-                int nn[4];
+                const int r = mi * 16 + 4 * q + j;
+                Lane &t = ts[mi][j];
+                float v[4];
 #pragma unroll
                 for (int ni = 0; ni < 4; ++ni) {
-                    const int n = n0 + ni * 16 + (lane & 15);
-                    nn[ni] = n;
-                    vv[ni] = -INFINITY;
-                    if (n >= NO) continue;
-                    const float v = acc[mi][ni][j] + a.b3[n];
-                    if (a.logits && r0 + r < a.batch) a.logits[(long long)(r0 + r) * NO + n] = v;
-                    if (n == a.C) stp[r] = v;
-                    else vv[ni] = v;
+                    v[ni] = acc[mi][ni][j] + bias[ni];
+                    const int n = g * 64 + ni * 16 + (lane & 15);
+                    if (a.logits && n < NO && r0 + r < a.batch) a.logits[(size_t)(r0 + r) * NO + n] = v[ni];
                 }
-                soft_add4(ts[mi][j], vv, nn);
+                if (whole) {
+                    // the sum's usual case -- finite values near the reference -- without a branch per value
+                    const float hi = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+                    const float lo = fminf(fminf(v[0], v[1]), fminf(v[2], v[3]));
+                    if (hi - t.ref <= REF_SPAN && lo >= -FLT_MAX) {
+#pragma unroll
+                        for (int ni = 0; ni < 4; ++ni) t.s += exp_mid(v[ni] - t.ref);
+                    } else {
+#pragma unroll
+                        for (int ni = 0; ni < 4; ++ni) lane_sum(t, v[ni]);
+                    }
+#pragma unroll
+                    for (int ni = 0; ni < 4; ++ni) lane_top(t, v[ni], g * 64 + ni * 16 + (lane & 15));
+                } else {
+#pragma unroll
+                    for (int ni = 0; ni < 4; ++ni) {
+                        const int n = g * 64 + ni * 16 + (lane & 15);
+                        if (n < a.C) {
+                            lane_sum(t, v[ni]);
+                            lane_top(t, v[ni], n);
+                        } else if (n == a.C) {
+                            stp[r] = v[ni];
+                        }
+                    }
+                }
             }
     }
+    // the 16 lanes of a row, then the waves
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int r = mi * 16 + 4 * (lane >> 4) + j;
-            Soft t = ts[mi][j];
+            const int r = mi * 16 + 4 * q + j;
+            const Lane &l = ts[mi][j];
+            Soft t{l.v1, l.v2, l.v1 == -INFINITY ? 0.0f : l.s * expf(l.ref - l.v1), l.a1, l.a2};
 #pragma unroll
             for (int o = 1; o < 16; o <<= 1) {
                 Soft u;
@@ -879,44 +899,65 @@ __global__ __launch_bounds__(IT) void infer_kernel(InferArgs a) {
     __syncthreads();
     if (tid < IQ) {
         Soft t = soft_empty();
-        for (int w = 0; w < IW; ++w) t = soft_merge(t, part[w * IQ + tid]);
+        for (int w = 0; w < WAVES; ++w) t = soft_merge(t, part[w * IQ + tid]);
         run[tid] = t;
     }
     __syncthreads();
-    // confidence: softmax mass of the best pivot's neighbourhood, its logits recomputed from
-    // the last hidden layer by TPR threads per row (entries e = quarter, quarter + TPR, ...);
-    // without neighbourhoods, the mass of the top two
+    // confidence: softmax mass of the best pivot's neighbourhood, its logits recomputed from the last
+    // hidden layer by the TPR threads of a row, eight hidden units at a time; without neighbourhoods,
+    // the mass of the top two
     {
-        constexpr int TPR = IT / IQ;
-        const int row = tid / TPR, quarter = tid % TPR;
-        const Soft t = run[row];
-        float mass = 0.0f;
-        if (a.nbr && t.a1 >= 0 && t.a1 < a.C) {  // (no valid best pivot: non-finite logits)
-            for (int e = quarter; e < a.n_nbr; e += TPR) {
-                const int p = a.nbr[(long long)t.a1 * a.n_nbr + e];
-                const uint16_t *w = a.W3 + (long long)p * a.hidden;
-                const uint16_t *hrow = H2 + row * ldh;
-                float z = a.b3[p];
-                for (int h = 0; h < a.hidden; h += 4) {
-                    const v4s wv = *reinterpret_cast<const v4s *>(w + h);
-                    const v4s hv = *reinterpret_cast<const v4s *>(hrow + h);
+        constexpr int TPR = IT >= 64 * IQ ? 64 : IT >= 32 * IQ ? 32 : IT >= 16 * IQ ? 16 : IT >= 8 * IQ ? 8 : 4;
+        const int row = tid / TPR, part_of = tid % TPR;
+        if (row < IQ) {
+            const Soft t = run[row];
+            float mass = 0.0f;
+            if (a.nbr && t.a1 >= 0 && t.a1 < a.C) {  // (no valid best pivot: non-finite logits)
+                for (int e = 0; e < a.n_nbr; ++e) {
+                    const int p = a.nbr[(size_t)t.a1 * a.n_nbr + e];
+                    const uint16_t *w = a.W3 + (size_t)p * a.hidden;
+                    float z = 0.0f;
+                    for (int h = part_of * 8; h < a.hidden; h += TPR * 8) {
+                        const uint4 wv = *reinterpret_cast<const uint4 *>(w + h);
+                        const uint4 hv = *reinterpret_cast<const uint4 *>(H2 + row * ldh + h);
+                        const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w}, hh[4] = {hv.x, hv.y, hv.z, hv.w};
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) z += bf2f((uint16_t)hv[q]) * bf2f((uint16_t)wv[q]);
+                        for (int u = 0; u < 4; ++u) {
+                            z += __uint_as_float(hh[u] << 16) * __uint_as_float(ww[u] << 16);
+                            z += __uint_as_float(hh[u] & 0xffff0000u) * __uint_as_float(ww[u] & 0xffff0000u);
+                        }
+                    }
+#pragma unroll
+                    for (int o = 1; o < TPR; o <<= 1) z += __shfl_xor(z, o);
+                    mass += expf(fminf(z + a.b3[p] - t.v1, 0.0f));
                 }
-                mass += expf(fminf(z - t.v1, 0.0f));
+            } else if (!a.nbr) {
+                mass = 1.0f + (t.v2 == -INFINITY ? 0.0f : expf(t.v2 - t.v1));
             }
-        } else if (!a.nbr && quarter == 0) {
-            mass = 1.0f + (t.v2 == -INFINITY ? 0.0f : expf(t.v2 - t.v1));
-        }
-#pragma unroll
-        for (int o = 1; o < TPR; o <<= 1) mass += __shfl_xor(mass, o);
-        if (quarter == 0 && r0 + row < a.batch) {
-            a.top2[2 * (r0 + row)] = t.a1;
-            a.top2[2 * (r0 + row) + 1] = t.a2;
-            a.conf[r0 + row] = fminf(mass / t.s, 1.0f);
-            a.stop[r0 + row] = stp[row];
+            if (part_of == 0 && r0 + row < a.batch) {
+                a.top2[2 * (r0 + row)] = t.a1;
+                a.top2[2 * (r0 + row) + 1] = t.a2;
+                a.conf[r0 + row] = fminf(mass / t.s, 1.0f);
+                a.stop[r0 + row] = stp[row];
+            }
         }
     }
+}
+
+template <int MI, int WAVES> static size_t infer_lds(const InferArgs &a) {
+    constexpr int IQ = 16 * MI;
+    const size_t ldh = (size_t)((a.hidden + 31) & ~31) + 8;
+    const size_t layers = (size_t)IQ * (a.width + 8 + ldh) * 2, soft = (size_t)(WAVES + 1) * IQ * sizeof(Soft);
+    return (size_t)IQ * ldh * 2 + IQ * 4 + std::max(layers, soft);
+}
+template <int MI, int WAVES> static int infer_launch(const InferArgs &a, hipStream_t st) {
+    constexpr int IQ = 16 * MI;
+    const size_t lds = infer_lds<MI, WAVES>(a);
+    if (lds > 65536)
+        MHIP(hipFuncSetAttribute((const void *)infer_kernel<MI, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL((infer_kernel<MI, WAVES>), dim3((a.batch + IQ - 1) / IQ), dim3(64 * WAVES), lds, st, a);
+    MHIP(hipGetLastError());
+    return 0;
 }
 
 // ---------------------------------------------------------------- host object
@@ -926,8 +967,10 @@ struct song_mlp {
     long long off[6] = {0}, cnt[6] = {0}, total = 0;  // W1 b1 W2 b2 W3 b3
     float *P = nullptr, *G = nullptr, *Mo = nullptr, *Vo = nullptr;
     uint16_t *Wb[3] = {nullptr, nullptr, nullptr};
-    uint16_t *W3i = nullptr;  // inference copy of the output weights, k-quad interleaved (infer_kernel)
-    int npad = 0;             // its column count: C + 1 rounded up to 16
+    uint16_t *W3i = nullptr;  // inference copy of the output weights (refresh_kernel)
+    int npad = 0;             // its column count: C + 1 rounded up to 64
+    int n_cu = 1;             // compute units of the device
+    size_t max_lds = 65536;
     int ldz = 0;              // row stride of Z and dZ: C + 1 rounded up to 8 (16-byte rows)
     uint16_t *H1 = nullptr, *H2 = nullptr, *dZ = nullptr, *dH2 = nullptr, *dH1 = nullptr;
     float *Z = nullptr, *loss = nullptr;
@@ -975,6 +1018,12 @@ extern "C" int song_mlp_create(int in_dim, int hidden, int n_classes, int max_ba
     m->hidden = hidden;
     m->C = n_classes;
     m->max_batch = max_batch;
+    int dev = 0;
+    hipDeviceProp_t prop;
+    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) {
+        m->n_cu = std::max(1, prop.multiProcessorCount);
+        m->max_lds = std::max<size_t>(65536, prop.sharedMemPerBlock);
+    }
     const long long sizes[6] = {(long long)hidden * m->width, hidden, (long long)hidden * hidden, hidden,
                                 (long long)(n_classes + 1) * hidden, n_classes + 1};
     long long o = 0;
@@ -1005,8 +1054,9 @@ extern "C" int song_mlp_create(int in_dim, int hidden, int n_classes, int max_ba
         return bad("params");
     for (int l = 0; l < 3; ++l)
         if (hipMalloc(&m->Wb[l], m->cnt[2 * l] * 2)) return bad("bf16 weights");
-    m->npad = (n_classes + 1 + 15) & ~15;
-    if (hipMalloc(&m->W3i, (size_t)m->npad * hidden * 2)) return bad("interleaved output weights");
+    m->npad = (n_classes + 1 + 63) & ~63;
+    const size_t w3i = (size_t)m->npad * ((hidden + 31) & ~31) * 2;
+    if (hipMalloc(&m->W3i, w3i) || hipMemset(m->W3i, 0, w3i)) return bad("interleaved output weights");
     m->ldz = (n_classes + 1 + 7) & ~7;
     const long long B = max_batch, LZ = m->ldz;
     if (hipMalloc(&m->H1, B * hidden * 2) || hipMalloc(&m->H2, B * hidden * 2) || hipMalloc(&m->dZ, B * LZ * 2) ||
@@ -1194,12 +1244,19 @@ extern "C" int song_mlp_infer_nbr(song_mlp *m, const uint16_t *d_x, int batch, c
     a.logits = d_logits;
     a.nbr = d_nbr;
     a.n_nbr = n_nbr;
-    const size_t lds = (size_t)IQ * (m->width + 8) * 2 + 2 * (size_t)IQ * (m->hidden + 8) * 2 +
-                       ((IW + 1) * IQ) * sizeof(Soft) + IQ * 4;
-    if (lds > 65536) MHIP(hipFuncSetAttribute((const void *)infer_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(infer_kernel, dim3((batch + IQ - 1) / IQ), dim3(IT), lds, (hipStream_t)stream, a);
-    MHIP(hipGetLastError());
-    return 0;
+    a.x16 = ((uintptr_t)d_x & 15) == 0;
+    // Block shape by how many 16-row tiles the batch has per compute unit.  Up to one each, a tile on 16
+    // waves is the shortest (33 rows: 47 us; on 8 waves 49, on 4 waves 113).  Beyond, two blocks of 8
+    // waves share a unit and take a tile each in about 67 us, or one block of 8 waves takes three tiles,
+    // each weight fragment serving three products, in 100 us: the cheaper of the two by whole rounds
+    // over the device (8,200-12,288 rows: 101 against 118 us; 6,000: 80 against 99; 60,000: 493 with
+    // one tile a block).
+    const long long t = (batch + 15) / 16, n = m->n_cu;
+    if (t <= n) return infer_launch<1, 16>(a, (hipStream_t)stream);
+    const long long rest = t % (2 * n);
+    const long long one = 67 * (t / (2 * n)) + (rest == 0 ? 0 : rest <= n ? 52 : 70), three = 100 * ((t + 3 * n - 1) / (3 * n));
+    if (three < one && infer_lds<3, 8>(a) <= m->max_lds) return infer_launch<3, 8>(a, (hipStream_t)stream);
+    return infer_launch<1, 8>(a, (hipStream_t)stream);
 }
 
 __global__ __launch_bounds__(256) void plan_kernel(const int *top2, const float *conf, const float *stop, int batch,
