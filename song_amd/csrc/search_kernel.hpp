@@ -21,19 +21,19 @@
 //   visited  : H slots, no deletion: compact 16-bit entries in groups of 8 (vis16_insert) or
 //              32-bit (id + 1) in groups of 4 (vis_insert), one 16-byte read per group; or,
 //              approximate, a blocked Bloom filter of 2^hlog 32-bit words (bloom_insert)
-//   best     : pq keys, sorted ascending, first nbest live (pq-best expanded list); absent
-//              with bglob, where the list's front lives in the wave slot's global region
+//   best     : pq keys, the front of the pq-best expanded list, in any order; absent with
+//              bglob, where the front lives in the wave slot's global region
 //   cid      : 256 u32   candidate ids of the current expansion / radix-select bins
 //   qv       : qld f32   the query, zero-padded to a multiple of 16
 // The queue head is one key per lane in registers, ascending over lanes [h, h + nq), nq <= 64.
 // The bag (qcap = pq + slack + 128 keys, unsorted, first bn live) is in global memory, one
 // region per wave slot: it is written by plain stores as candidates arrive and read only when
 // the head runs empty or the bag nears its capacity, so LDS holds only what every step
-// touches and more waves fit on a CU.  The best list's last 64 positions are one key per lane
-// in registers; its front (the first nbest - 64) is written once per entry while the list
-// grows and read only when an expansion lands below the register tail, which is rare, and at
-// the end -- so with bglob it lives after the bag in the slot's global region (pq keys) and a
-// large pq does not cost LDS.
+// touches and more waves fit on a CU.  The best list's 64 largest entries are one key per lane
+// in registers; its front (the others, unsorted) is written once per entry and read only when
+// 64 expansions have landed below the tail of a full list, and at the end, where the results
+// are selected from it -- so with bglob it lives after the bag in the slot's global region (pq
+// keys) and a large pq does not cost LDS.
 //
 // Each wave owns its LDS slice (one wave per workgroup in search_kernel; 1-4 waves, each
 // on its own slice, in search_persistent).  LDS instructions of a wave execute in issue
@@ -700,50 +700,12 @@ __device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, con
     return mine;
 }
 
-// wave-wide minimum of a KeyF (all lanes get it)
-__device__ __forceinline__ KeyF wave_min(KeyF k) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint64_t v = ((uint64_t)(uint32_t)__shfl_xor((int)(k.v >> 32), o) << 32) |
-                           (uint32_t)__shfl_xor((int)k.v, o);
-        if (v < k.v) k.v = v;
-    }
-    return k;
-}
-
-// Count of the leading entries of the sorted run arr[0..n) that satisfy `below`, a
-// predicate that holds on a prefix.  64-ary search: each round samples the last entry of
-// 64 equal chunks (one LDS read per lane) and keeps the chunk holding the boundary.
-template <class Key, class Pred>
-__device__ __forceinline__ int prefix_count(const Key *arr, int n, Pred below) {
+// entries of arr[0..n), in any order, below x
+template <class Key> __device__ __forceinline__ int count_below(const Key *arr, int n, const Key &x) {
     const int lane = rare_lane();
-    int lo = 0, len = n;
-    while (len > 64) {
-        const int stride = (len + 63) >> 6;
-        const int end = lo + len;
-        const int idx = min(lo + (lane + 1) * stride, end) - 1;
-        const bool v = lo + lane * stride < end;
-        const Key e = arr[v ? idx : lo];
-        const int c = __popcll(ballot(v && below(e)));
-        lo = min(lo + c * stride, end);  // the last chunk may be partial
-        len = min(stride, end - lo);
-    }
-    const bool v = lane < len;
-    const Key e = arr[v ? lo + lane : 0];
-    return lo + __popcll(ballot(v && below(e)));
-}
-
-// arr[p, e) moves to arr[p + 1, e + 1) and arr[p] = x (blocks of 64, last block first, so each
-// block is read before the block below it writes into its first slot)
-template <class Key> __device__ __forceinline__ void shift_insert(Key *arr, int p, int e, const Key &x) {
-    const int lane = rare_lane();
-    for (int blk = (e - 1) >> 6; blk >= (p >> 6) && e > p; --blk) {
-        const int i = blk * 64 + lane;
-        const bool live = i >= p && i < e;
-        const Key v = arr[live ? i : 0];
-        if (live) arr[i + 1] = v;
-    }
-    if (lane == 0) arr[p] = x;
+    int c = 0;
+    for (int b0 = 0; b0 < n; b0 += 64) c += __popcll(ballot(b0 + lane < n && lt(arr[b0 + lane], x)));
+    return c;
 }
 
 // ---------------------------------------------------------------- wave-wide key sets
@@ -755,6 +717,9 @@ __device__ __forceinline__ KeyD shfl_key(const KeyD &k, int src) {
     return KeyD{((uint64_t)(uint32_t)__shfl((int)(k.d >> 32), src) << 32) | (uint32_t)__shfl((int)k.d, src),
                 (uint32_t)__shfl((int)k.i, src), 0u};
 }
+// the key order reversed (-> +inf, the largest key, only from the smallest possible one)
+__device__ __forceinline__ KeyF flip(const KeyF &k) { return KeyF{~k.v}; }
+__device__ __forceinline__ KeyD flip(const KeyD &k) { return KeyD{~k.d, ~k.i, 0u}; }
 template <class Key> __device__ __forceinline__ Key kmin(const Key &a, const Key &b) { return lt(b, a) ? b : a; }
 template <class Key> __device__ __forceinline__ Key kmax(const Key &a, const Key &b) { return lt(b, a) ? a : b; }
 
@@ -778,15 +743,17 @@ __device__ __forceinline__ Key bitonic_steps(Key v, int K, int J) {
 // merged: min(best[i], block[63 - i]) holds the 64 smallest of both as a bitonic sequence.
 // Bags are appended in nearly ascending order, so most blocks after the first are skipped or
 // take a few insertions.
+// FLIP: of the reversed order (the largest keys, reversed, the largest first).
 constexpr int SEL_INSERT = 16;
-template <class Key>
+template <bool FLIP = false, class Key>
 __device__ __forceinline__ Key select64(const Key *arr, int n) {
     const int lane = rare_lane();
-    Key best = (lane < n) ? arr[lane] : Key::inf();
+    const auto at = [&](int i) __attribute__((always_inline)) { return i < n ? (FLIP ? flip(arr[i]) : arr[i]) : Key::inf(); };
+    Key best = at(lane);
     // two blocks' loads are in flight while one is sorted or scanned (two register slots, the
     // loop unrolled by two, so no slot is copied while its load is in flight)
-    Key na = (64 + lane < n) ? arr[64 + lane] : Key::inf();
-    Key nb = (128 + lane < n) ? arr[128 + lane] : Key::inf();
+    Key na = at(64 + lane);
+    Key nb = at(128 + lane);
     for (int k = 2; k <= 64; k <<= 1) best = bitonic_steps(best, k, k);
     const auto take = [&](Key v) {
         uint64_t m = ballot(lt(v, best.rl(63)));
@@ -805,11 +772,11 @@ __device__ __forceinline__ Key select64(const Key *arr, int n) {
     };
     for (int b0 = 64; b0 < n; b0 += 128) {
         const Key va = na;
-        if (b0 + 128 < n) na = (b0 + 128 + lane < n) ? arr[b0 + 128 + lane] : Key::inf();
+        if (b0 + 128 < n) na = at(b0 + 128 + lane);
         take(va);
         if (b0 + 64 < n) {
             const Key vb = nb;
-            if (b0 + 192 < n) nb = (b0 + 192 + lane < n) ? arr[b0 + 192 + lane] : Key::inf();
+            if (b0 + 192 < n) nb = at(b0 + 192 + lane);
             take(vb);
         }
     }
@@ -1065,12 +1032,14 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     uint32_t nglob = 0u;
     uint32_t *gv = nullptr;
     const uint32_t GH = 1u << P.ghlog, gmask = GH - 1u, glimit = (GH >> 2) * 3u;
-    int h = 0, nq = 0, nbest = 0;
-    uint64_t bmax = ~0ull;  // distance key of best[pq-1] once the list is full
-    // the best list's last positions [tb, tb + 64) live in registers: lane j holds position
-    // tb + j (+inf past nbest); the front [0, tb) is in LDS.  tb = max(0, nbest - 64).
+    int h = 0, nq = 0;
+    // The best list (the pq smallest expanded keys): its largest nt <= 64 entries, the tail, ascending in
+    // lanes [0, nt) of a register (+inf above), the other nf, the front, in memory in any order.  Only the
+    // list's largest entry matters to the search, and expansions come out in nearly ascending order, so
+    // almost all of them end in the tail; one below it is appended to the front.
     Key bt = Key::inf();
-    int tb = 0;
+    int nt = 0, nf = 0;
+    uint64_t bmax = ~0ull;  // distance key of the largest entry once the list is full
     // the queue head lives in registers: lanes [h, h + nq) hold its keys in ascending order
     Key hq = Key::inf();
     int bn = 0;          // bag entries: unsorted, all above T
@@ -1174,7 +1143,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         }
         const Key now = hq.rl(h);
         // stop rule, graph.h:188: |best| == pq and best.max.d < now.d (distance only, strict)
-        if (nbest == pq && bmax < now.dk()) return true;
+        if (nf + nt == pq && bmax < now.dk()) return true;
         ++steps;
         ++h;
         --nq;
@@ -1196,48 +1165,57 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         prow[Y] = adj_row(nq > 0 ? pid[Y] : 0u);
         if (nq > 0) publish(pid[Y]);
 
-        // insert `now` into the sorted pq-best list (push + pop-max of graph.h:193-195).
-        // Expansions come out in nearly ascending order, so `now` almost always lands in the
-        // register tail: one compare and a lane shift, no LDS round trip.
+        // `now` into the pq-best list (push + pop-max of graph.h:193-195).  A sorted front cost a search
+        // and a shift through memory for every expansion below the tail: 10,000 queries at pq 704 took
+        // 12.57 ms with it and take 9.75 ms without (front in global memory; 14.1 and 12.8 ms in LDS).
         {
             // the tail's entries below `now` are its first c lanes, so the ballot itself is the mask of the
             // lanes that keep their entry
             const uint64_t below = ballot(lt(bt, now));
-            int p = tb + __popcll(below);
-            if (tb > 0 && !(below & 1ull)) {  // below the tail: in the front, or right at the tail's start
-                front_fence();
-                p = prefix_count(Bf(), tb, [&](const Key &e) { return lt(e, now); });
-            }
-            if (p < k && lane == 0) settle = steps;
-            if (p < pq) {
-                if (p >= tb) {
-                    const int c = p - tb;
-                    if (nbest >= 64 && nbest < pq) {
-                        // growing past 64 entries: the smallest of the 65 entries [tb, nbest] with `now`
-                        // at c goes to the front, lanes below c - 1 take their upper neighbour's entry
-                        if (lane == 0) Bf()[tb] = ksel(c == 0, now, bt);
-                        bt = ksel(in_mask(below >> 1), shl1(bt), bt);
-                        if (c > 0) bt = ksel(in_mask(1ull << (c - 1)), now, bt);
-                        ++tb;
-                    } else {
-                        // below 64 entries (tb = 0), or full (the entry at pq - 1 leaves)
-                        bt = ksel(in_mask(below), bt, shr1(bt));
-                        bt = ksel(in_mask(1ull << c), now, bt);
-                        if (nbest == pq && pq < 64) bt = ksel(in_mask(1ull << pq), Key::inf(), bt);
-                    }
-                } else if (nbest < pq) {
-                    // front [p, tb) moves to [p + 1, tb + 1); the tail keeps its entries
-                    shift_insert(Bf(), p, tb, now);  // (a front in global memory: after the fence above)
-                    ++tb;
-                } else {
-                    // full: the front's last entry moves into the tail, the entry at pq - 1 leaves
-                    const Key fl = Bf()[tb - 1];
-                    shift_insert(Bf(), p, tb - 1, now);
-                    const Key dn = shr1(bt);
-                    bt = ksel(lane == 0, fl, dn);
+            const int c = __popcll(below);
+            const bool full = nf + nt == pq;
+            const bool in_tail = c > 0 || nf == 0;  // at or above the tail's smallest, or all is tail
+            if (P.out_stats) {
+                // the first k results change when fewer than k entries are smaller
+                int p = nf + c;
+                if (!in_tail) {
+                    front_fence();
+                    p = count_below(Bf(), nf, now);
                 }
-                nbest = min(nbest + 1, pq);
-                if (nbest == pq) bmax = bt.rl(pq - 1 - tb).dk();
+                if (p < k && lane == 0) settle = steps;
+            }
+            if (!full || c < nt) {
+                if (in_tail && (full || nt < 64)) {
+                    // lanes from c on move up one; of a full list the largest entry leaves
+                    bt = ksel(in_mask(below), bt, shr1(bt));
+                    bt = ksel(in_mask(1ull << c), now, bt);
+                    if (!full) ++nt;
+                    else if (nt < 64) bt = ksel(in_mask(1ull << nt), Key::inf(), bt);
+                } else {
+                    // a key joins the front: `now` if it is below the tail, else the tail's smallest, the
+                    // lanes below c - 1 taking their upper neighbour's entry and `now` lane c - 1
+                    if (lane == 0) Bf()[nf] = ksel(c == 0, now, bt);
+                    ++nf;
+                    if (c > 0) {
+                        bt = ksel(in_mask(below >> 1), shl1(bt), bt);
+                        bt = ksel(in_mask(1ull << (c - 1)), now, bt);
+                    } else if (full) {
+                        --nt;  // the largest entry leaves
+                        bt = ksel(in_mask(1ull << nt), Key::inf(), bt);
+                        if (nt == 0) {
+                            // the front's largest entries become the tail
+                            front_fence();
+                            const Key sel = select64<true>(Bf(), nf);
+                            nt = min(64, nf);
+                            bt = flip(shfl_key(sel, (nt - 1 - lane) & 63));
+                            bt = ksel(in_mask(low_bits(nt)), bt, Key::inf());
+                            const Key low = bt.rl(0);
+                            nf = compact(Bf(), nf, [&](const Key &e) { return lt(e, low); });
+                            if constexpr (BG) vm_drain();
+                        }
+                    }
+                }
+                if (nf + nt == pq) bmax = bt.rl(nt - 1).dk();
                 lds_fence();
             }
         }
@@ -1319,14 +1297,14 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         if (!cached) mine = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m, cid, qv, lenv);
 
         // ---- the candidates: at most T into the sorted head, above T into the bag
-        const uint64_t cut = (nbest == pq) ? bmax : ~0ull;  // drop distance keys above cut
+        const uint64_t cut = (nf + nt == pq) ? bmax : ~0ull;  // drop distance keys above cut
         const bool surv = have && mine.dk() <= cut;
         if (ballot(surv) == 0ull) return false;
         // (a row has at most 63 neighbours, each of which adds at most one key to the bag)
         if (bn + 63 > P.qcap) {
             // make room: drop bag entries beyond the pq-th smallest distance of head + bag
             // (ties kept) or beyond bmax; none of them can be expanded before the stop rule
-            uint64_t dcut = (nbest == pq) ? bmax : ~0ull;
+            uint64_t dcut = (nf + nt == pq) ? bmax : ~0ull;
             truncs += l0;
             if constexpr (BAGL) lds_fence(); else bag_fence();
             if (pq <= nq) dcut = min(dcut, hq.rl(h + pq - 1).dk());
@@ -1359,16 +1337,16 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     }
     // the whole best list in LDS (or, bglob, in the slot's global region) from here on
     if constexpr (BG) B = Bf();
-    if (lane < nbest - tb) B[tb + lane] = bt;
+    if (lane < nt) B[nf + lane] = bt;
+    const int nbest = nf + nt;
     if constexpr (BG) bag_fence();
     else lds_fence();
 
     const int cnt = min(k, nbest);
     const size_t ob = (size_t)qi * (size_t)P.out_ld;
-    bool done = false;
     if constexpr (STORE != ST_F32 && !EXACT) {
         if (P.rerank) {
-            // exact FP32 distances for the whole pq-best list, then the k smallest in order
+            // exact FP32 distances for the whole pq-best list
             for (int base = 0; base < nbest; base += 64) {
                 const int c = min(64, nbest - base);
                 if (lane < c) cid[lane] = B[base + lane].id();
@@ -1377,34 +1355,25 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
                 if (cand_of_lane<4>() < c) B[base + cand_of_lane<4>()] = ex;
                 lds_fence();
             }
-            for (int r = 0; r < k; ++r) {
-                Key best = Key::inf();
-                int bi = -1;
-                for (int i = lane; i < nbest; i += 64) {
-                    const Key e = B[i];
-                    if (lt(e, best)) {
-                        best = e;
-                        bi = i;
-                    }
-                }
-                const Key w = wave_min(best);
-                if (bi >= 0 && best.v == w.v) B[bi] = Key::inf();
-                lds_fence();
-                if (lane == 0) {
-                    const bool ok = r < cnt;
-                    P.out_ids[ob + r] = ok ? w.id() : 0xFFFFFFFFu;
-                    if (P.out_dist) P.out_dist[ob + r] = ok ? w.dist() : __int_as_float(0x7f800000);
-                }
-            }
-            done = true;
         }
     }
-    // output: first k of the ascending list (graph.h:209-215)
-    for (int i = lane; i < k && !done; i += 64) {
-        const bool ok = i < cnt;
-        const Key e = ok ? B[i] : Key::inf();
-        P.out_ids[ob + i] = ok ? e.id() : 0xFFFFFFFFu;
-        if (P.out_dist) P.out_dist[ob + i] = ok ? e.dist() : __int_as_float(0x7f800000);
+    // output: the first k in ascending order (graph.h:209-215), 64 at a time
+    for (int i0 = 0, n = nbest; i0 < k; i0 += 64) {
+        Key e = Key::inf();
+        if (i0 < cnt) {
+            e = select64(B, n);
+            if (i0 + 64 < cnt) {
+                n = keep_above(B, n, e.rl(63));
+                if constexpr (BG) bag_fence();
+                else lds_fence();
+            }
+        }
+        const int i = i0 + lane;
+        if (i < k) {
+            const bool ok = i < cnt;
+            P.out_ids[ob + i] = ok ? e.id() : 0xFFFFFFFFu;
+            if (P.out_dist) P.out_dist[ob + i] = ok ? e.dist() : __int_as_float(0x7f800000);
+        }
     }
     if (lane == 0) {
         if (P.retry_list && (flags & (F_VIS_OVF | F_Q_OVF))) P.retry_list[atomicAdd(P.retry_count, 1u)] = (uint32_t)qi;
