@@ -355,7 +355,7 @@ __device__ __forceinline__ int vis16_insert(uint32_t *vis, int gbits, int idbits
         r = atomicCAS(&grp[wi], old, nw) == old ? 1 : 2;
         lds_fence();
     }
-    if (r == 2) r = vis16_probe(vis, gbits, home, lo1);
+    if (r == 2) [[unlikely]] r = vis16_probe(vis, gbits, home, lo1);
     return r;
 }
 __device__ __forceinline__ bool vis16_test(const uint32_t *vis, int gbits, int idbits, uint32_t id) {
@@ -410,6 +410,7 @@ __device__ __forceinline__ uint32_t bloom_mask(uint32_t h1, uint32_t h2, int k) 
     return m;
 }
 __device__ __forceinline__ bool bloom_insert(uint32_t *bf, int wlog, int k, uint32_t id) {
+    asm volatile("" : "+s"(k));  // its nine compares belong here, not hoisted out of the search loop
     const uint32_t h1 = fmix32(id * 2u + 1u), h2 = fmix32(id ^ 0x9E3779B9u);
     const uint32_t mask = bloom_mask(h1, h2, k);
     const uint32_t old = atomicOr(&bf[h1 >> (32 - wlog)], mask);
@@ -1028,9 +1029,21 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     uint32_t adj_words = 0u, pf_hits = 0u, refills = 0u, truncs = 0u;
     const uint32_t l0 = lane == 0 ? 1u : 0u;
     // visited spill: once the LDS table nears its load limit, new ids go to a global table
-    bool spill = false;
+    // vmode: what an id is tested against -- the compact or the 32-bit LDS table, the Bloom filter, or
+    // (after the switch) an LDS table and the global one
+    enum { V_16 = 0, V_32 = 1, V_BLOOM = 2, V_SPILL = 3 };
+    int vmode = bloom ? V_BLOOM : P.vis16 ? V_16 : V_32;
+    uint32_t vstop = bloom ? ~0u : vis_limit - 64u;  // vertices beyond which the table switches
     uint32_t nglob = 0u;
     uint32_t *gv = nullptr;
+    // the rest of this query's new ids go to the slot's global table, cleared here
+    const auto to_spill = [&]() __attribute__((always_inline)) {
+        vmode = V_SPILL;
+        vstop = ~0u;
+        gv = P.gvis + (size_t)slot_q * (1u << P.ghlog);
+        for (uint32_t i = (uint32_t)rare_lane(); i < (1u << P.ghlog); i += 64) gv[i] = 0u;
+        __threadfence_block();
+    };
     const uint32_t GH = 1u << P.ghlog, gmask = GH - 1u, glimit = (GH >> 2) * 3u;
     int h = 0, nq = 0;
     // The best list (the pq smallest expanded keys): its largest nt <= 64 entries, the tail, ascending in
@@ -1121,12 +1134,12 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     // one expansion; returns true to leave the loop
     const auto expand = [&](auto parity) -> bool {
         constexpr int X = decltype(parity)::value, Y = 1 - X;
-        if (nq == 0 && bn == 0) return true;
-        if (steps >= max_steps) {
+        if (nq == 0 && bn == 0) [[unlikely]] return true;
+        if (steps >= max_steps) [[unlikely]] {
             flags |= F_STEP_CAP;
             return true;
         }
-        if (nq == 0) {
+        if (nq == 0) [[unlikely]] {
             // refill the head with the (up to) 64 smallest bag entries
             const int c = min(QH, bn);
             refills += l0;
@@ -1143,14 +1156,14 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         }
         const Key now = hq.rl(h);
         // stop rule, graph.h:188: |best| == pq and best.max.d < now.d (distance only, strict)
-        if (nf + nt == pq && bmax < now.dk()) return true;
+        if (nf + nt == pq && bmax < now.dk()) [[unlikely]] return true;
         ++steps;
         ++h;
         --nq;
 
         // adjacency row of `now`: slot X holds it when the prefetch predicted this vertex;
         // otherwise it is loaded into slot X now
-        if (pid[X] == now.id()) {
+        if (pid[X] == now.id()) [[likely]] {
             pf_hits += l0;
         } else {
             pid[X] = now.id();
@@ -1175,7 +1188,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
             const int c = __popcll(below);
             const bool full = nf + nt == pq;
             const bool in_tail = c > 0 || nf == 0;  // at or above the tail's smallest, or all is tail
-            if (P.out_stats) {
+            if (P.out_stats) [[unlikely]] {
                 // the first k results change when fewer than k entries are smaller
                 int p = nf + c;
                 if (!in_tail) {
@@ -1202,7 +1215,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
                     } else if (full) {
                         --nt;  // the largest entry leaves
                         bt = ksel(in_mask(1ull << nt), Key::inf(), bt);
-                        if (nt == 0) {
+                        if (nt == 0) [[unlikely]] {
                             // the front's largest entries become the tail
                             front_fence();
                             const Key sel = select64<true>(Bf(), nf);
@@ -1223,53 +1236,45 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         // neighbours of `now` in row order (graph.h:196-205)
         const int deg = (int)rl32(r, 0);
         adj_words += l0 * (1u + (uint32_t)deg);
-        if (!bloom && !spill && nvis + 64u > vis_limit) {
+        if (nvis > vstop) [[unlikely]] {
             if (!P.gvis) {
                 flags |= F_VIS_OVF;
                 return true;
             }
-            // switch to the global table for the rest of this query: clear it first
-            spill = true;
-            gv = P.gvis + (size_t)slot_q * GH;
-            for (uint32_t i = lane; i < GH; i += 64) gv[i] = 0u;
-            __threadfence_block();
+            to_spill();
         }
-        bool fresh = false, vovf = false;
-        if (lane >= 1 && lane <= deg) {
-            if (bloom) {
-                fresh = bloom_insert(vis, P.hlog, P.bloom_k, r);
-            } else if (!spill) {
-                if (P.vis16) {
-                    const int ins = vis16_insert(vis, gbits, P.idbits, r);
-                    fresh = ins == 1;
-                    vovf = ins == 2;
-                } else {
-                    fresh = vis_insert(vis, hmask, P.hlog, r);
+        bool fresh = false;
+        const uint64_t nb = low_bits(deg + 1) & ~1ull;  // lanes 1..deg hold the neighbours
+        if (vmode == V_16) [[likely]] {
+            bool vovf = false;
+            if (in_mask(nb)) {
+                const int ins = vis16_insert(vis, gbits, P.idbits, r);
+                fresh = ins == 1;
+                vovf = ins == 2;
+            }
+            if (ballot(vovf) != 0ull) [[unlikely]] {
+                // the compact table had no room near these ids: continue in the global table
+                if (!P.gvis) {
+                    flags |= F_VIS_OVF;
+                    return true;
                 }
-            } else {
-                const bool in_lds = P.vis16 ? vis16_test(vis, gbits, P.idbits, r) : vis_test(vis, hmask, P.hlog, r);
-                fresh = !in_lds && gvis_insert(gv, gmask, P.ghlog, r);
+                to_spill();
+                if (vovf) fresh = gvis_insert(gv, gmask, P.ghlog, r);
             }
-        }
-        if (!bloom && P.vis16 && ballot(vovf) != 0ull) {
-            // the compact table had no room near these ids: continue in the global table
-            if (!P.gvis) {
-                flags |= F_VIS_OVF;
-                return true;
-            }
-            if (!spill) {
-                spill = true;
-                gv = P.gvis + (size_t)slot_q * GH;
-                for (uint32_t i = lane; i < GH; i += 64) gv[i] = 0u;
-                __threadfence_block();
-            }
-            if (vovf) fresh = gvis_insert(gv, gmask, P.ghlog, r);
+        } else if (vmode == V_32) {
+            if (in_mask(nb)) fresh = vis_insert(vis, hmask, P.hlog, r);
+        } else if (vmode == V_BLOOM) {
+            if (in_mask(nb)) fresh = bloom_insert(vis, P.hlog, P.bloom_k, r);
+        } else {
+            bool in_lds = true;
+            if (in_mask(nb)) in_lds = P.vis16 ? vis16_test(vis, gbits, P.idbits, r) : vis_test(vis, hmask, P.hlog, r);
+            if (!in_lds) fresh = gvis_insert(gv, gmask, P.ghlog, r);
         }
         const uint64_t fm = ballot(fresh);
         const int m = __popcll(fm);
         if (fresh) cid[lanes_below(fm)] = r;
         nvis += (uint32_t)m;
-        if (spill) {
+        if (vmode == V_SPILL) [[unlikely]] {
             nglob += (uint32_t)m;
             if (nglob + 64u > glimit) {
                 flags |= F_VIS_OVF;
@@ -1301,7 +1306,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         const bool surv = have && mine.dk() <= cut;
         if (ballot(surv) == 0ull) return false;
         // (a row has at most 63 neighbours, each of which adds at most one key to the bag)
-        if (bn + 63 > P.qcap) {
+        if (bn + 63 > P.qcap) [[unlikely]] {
             // make room: drop bag entries beyond the pq-th smallest distance of head + bag
             // (ties kept) or beyond bmax; none of them can be expanded before the stop rule
             uint64_t dcut = (nf + nt == pq) ? bmax : ~0ull;
