@@ -1118,13 +1118,14 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     const int max_steps = P.steps_arr ? min(P.steps_arr[qi], P.max_steps) : P.max_steps;
     int settle = 0;  // lane 0 holds it
 
-    // adjacency rows loaded one expansion ahead, in two slots used in turn: an expansion of
-    // parity X reads its row from slot X where it lies and loads the next head's row into slot
-    // Y, whose row the previous expansion has consumed.  No row is copied between registers, so
-    // nothing waits for a load before the row is first used (a copy of a register whose load is
-    // in flight waits for that load).  The loop body is instantiated once per parity.
+    // The adjacency row of the next expansion is asked for twice: `ahead`, of the predicted next vertex
+    // right after the pop, a whole expansion early, which brings it into the caches; and `row`, of the
+    // queue head when the expansion ends, which is the one used (nearly always the same row: a cache
+    // hit that is there after the next pop).  Both loads are issued on every expansion and neither
+    // register is written anywhere else on the common path, so no copy of a register whose load is in
+    // flight -- which waits for that load, and for the bag's stores before it -- is ever needed.
     constexpr uint32_t NONE = 0xFFFFFFFFu;
-    uint32_t pid[2] = {NONE, NONE}, prow[2] = {0u, 0u};
+    uint32_t row_id = NONE, row = 0u, ahead = 0u;
     // all lanes load (lanes past the row read its last word and are never used: a row's
     // degree is below gstride), so the load needs no lane mask and no zero fill
     const auto adj_row = [&](uint32_t v) -> uint32_t {
@@ -1132,8 +1133,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     };
 
     // one expansion; returns true to leave the loop
-    const auto expand = [&](auto parity) -> bool {
-        constexpr int X = decltype(parity)::value, Y = 1 - X;
+    const auto expand = [&]() -> bool {
         if (nq == 0 && bn == 0) [[unlikely]] return true;
         if (steps >= max_steps) [[unlikely]] {
             flags |= F_STEP_CAP;
@@ -1151,7 +1151,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
             nq = c;
             bn = keep_above(Bg, bn, top);
             T = bn > 0 ? top : Key::inf();
-            pid[X] = NONE;
+            row_id = NONE;
             if constexpr (!BAGL) vm_drain();
         }
         const Key now = hq.rl(h);
@@ -1161,22 +1161,17 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         ++h;
         --nq;
 
-        // adjacency row of `now`: slot X holds it when the prefetch predicted this vertex;
-        // otherwise it is loaded into slot X now
-        if (pid[X] == now.id()) [[likely]] {
+        if (row_id == now.id()) [[likely]] {
             pf_hits += l0;
         } else {
-            pid[X] = now.id();
-            prow[X] = adj_row(now.id());
+            row = adj_row(now.id());
         }
-        const uint32_t r = prow[X];
-        // prefetch the row of the new queue head, the likely next expansion, into slot Y.  The
-        // load is issued on every expansion (vertex 0's row when the head is empty) so that a
-        // load always follows this expansion's row: the wait before the row's first use then
-        // leaves the prefetch in flight.
-        pid[Y] = nq > 0 ? hq.rl(h).id() : NONE;
-        prow[Y] = adj_row(nq > 0 ? pid[Y] : 0u);
-        if (nq > 0) publish(pid[Y]);
+        const uint32_t r = row;
+        // (vertex 0's row when the head is empty: the load is issued on every expansion)
+        const uint32_t next_id = nq > 0 ? hq.rl(h).id() : 0u;
+        asm volatile("" ::"v"(ahead));  // the previous `ahead` has come in before `row` did
+        ahead = adj_row(next_id);
+        if (nq > 0) publish(next_id);
 
         // `now` into the pq-best list (push + pop-max of graph.h:193-195).  A sorted front cost a search
         // and a shift through memory for every expansion below the tail: 10,000 queries at pq 704 took
@@ -1328,17 +1323,14 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         if (to_b) Bg[bn + lanes_below(bm)] = mine;
         bn += __popcll(bm);
         for (uint64_t bits = ballot(to_q); bits; bits &= bits - 1) push_head(mine.rl(__builtin_ctzll(bits)));
-        // the queue head may have changed: refresh the prefetch target only if it did
-        if (nq > 0 && hq.rl(h).id() != pid[Y]) {
-            pid[Y] = hq.rl(h).id();
-            prow[Y] = adj_row(pid[Y]);
-            publish(pid[Y]);
-        }
+        // the helper's target follows the queue head
+        if constexpr (HELP)
+            if (nq > 0 && hq.rl(h).id() != next_id) publish(hq.rl(h).id());
         return false;
     };
-    for (;;) {
-        if (flags != 0u || expand(std::integral_constant<int, 0>{})) break;
-        if (expand(std::integral_constant<int, 1>{})) break;
+    while (flags == 0u && !expand()) {
+        row_id = nq > 0 ? hq.rl(h).id() : NONE;
+        row = adj_row(nq > 0 ? row_id : 0u);
     }
     // the whole best list in LDS (or, bglob, in the slot's global region) from here on
     if constexpr (BG) B = Bf();
