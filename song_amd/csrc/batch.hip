@@ -382,6 +382,9 @@ static int enqueue(song_batch *b, const RunArgs &a, hipStream_t st) {
     sp.dim = ix->dim;
     sp.ld = ix->ld;
     sp.gstride = ix->gstride;
+    sp.int_rows = ix->integer_valued;
+    sp.row_min = ix->vmin;
+    sp.row_max = ix->vmax;
     sp.nq = (int)a.nq;
     sp.k = a.k;
     sp.out_ld = a.k_ld;

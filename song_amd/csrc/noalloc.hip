@@ -153,6 +153,9 @@ extern "C" int song_search_device_noalloc(song_index *ix, const float *d_queries
     sp.dim = ix->dim;
     sp.ld = ix->ld;
     sp.gstride = ix->gstride;
+    sp.int_rows = ix->integer_valued;
+    sp.row_min = ix->vmin;
+    sp.row_max = ix->vmax;
     sp.nq = (int)nq;
     sp.pq = pq;
     sp.k = k;

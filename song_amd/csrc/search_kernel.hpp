@@ -25,7 +25,8 @@
 //              bglob, where the front lives in the wave slot's global region
 //   cid      : 256 u32   candidate ids of the current expansion / radix-select bins
 //   qv       : qld f32   the query, zero-padded to a multiple of 16
-// The queue head is one key per lane in registers, ascending over lanes [h, h + nq), nq <= 64.
+// The queue head is one key per lane in registers, ascending over lanes [h, h + nq), nq <= 64,
+// +inf in the others.
 // The bag (qcap = pq + slack + 128 keys, unsorted, first bn live) is in global memory, one
 // region per wave slot: it is written by plain stores as candidates arrive and read only when
 // the head runs empty or the bag nears its capacity, so LDS holds only what every step
@@ -106,6 +107,8 @@ struct SearchParams {
                             // bloom_k bits per id in one word (approximate: false positives skip vertices)
     int multiprobe;         // several-queries-per-wave kernel: expansions per step (1, or 2: the next
                             // queue head too; approximate)
+    int int_rows;           // 1: every row value is an integer, in [row_min, row_max]
+    float row_min, row_max;
 };
 
 // bytes of a slot's bag before the best-list front (bglob): qcap keys rounded to 256
@@ -174,9 +177,10 @@ __device__ __forceinline__ KeyF rl_key(const KeyF &k, int lane) { return k.rl(la
 __device__ __forceinline__ KeyD rl_key(const KeyD &k, int lane) { return k.rl(lane); }
 
 // whole-wave lane shifts by one (DPP wave_shl:1 / wave_shr:1): shl1 gives lane i the value of
-// lane i + 1 (lane 63 keeps its own), shr1 the value of lane i - 1 (lane 0 keeps its own)
+// lane i + 1 (lane 63 gets 0), shr1 the value of lane i - 1 (lane 0 gets 0).  The end lane's value is
+// left to the instruction (zero), not to a copy made first; no caller uses it.
 template <int CTRL> __device__ __forceinline__ uint32_t dpp32(uint32_t x) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xF, 0xF, false);
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xF, 0xF, true);
 }
 constexpr int DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138;
 template <int CTRL> __device__ __forceinline__ uint64_t dpp64(uint64_t x) {
@@ -694,7 +698,7 @@ __device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, con
         if (redo) {
             const uint32_t id = mine.id();
             const float lena = (METRIC == M_COS) ? P.norms[id] : 0.0f;
-            const double s = seq_sum<METRIC, (SUB >= 16 ? 8 : 1)>(P.data + (size_t)id * (size_t)P.ld, qv, P.dim);
+            const double s = seq_sum<METRIC, (SUB * NVU > 64 ? 8 : 1)>(P.data + (size_t)id * (size_t)P.ld, qv, P.dim);
             mine = Key::make_d(finish_exact<METRIC>(s, lena, lenv), id);
         }
     }
@@ -766,7 +770,7 @@ __device__ __forceinline__ Key select64(const Key *arr, int n) {
                 const Key x = v.rl(__builtin_ctzll(m));
                 // rank 64 (x above the current 64th, lowered by earlier insertions): no change
                 const int r = __popcll(ballot(lt(best, x)));
-                const Key dn = shr1(best);
+                const Key dn = shr1(best);  // (lane 0's is not used: it keeps its key or takes x)
                 best = ksel(lane < r, best, ksel(lane == r, x, dn));
             }
         }
@@ -987,6 +991,33 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         lenv = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(lenv)));
     }
 
+    // May a distance be summed in any order?  In exact mode always (a sum is exact in any order, or done
+    // again in the CPU's); with float sums when rows and query are integers and every partial sum is
+    // below 2^24.  Then up to 4 candidates take 16 lanes a row in place of Shape's 4: a quarter of the
+    // row's serial work per lane, the same sums.
+    constexpr bool WIDE = SUB == 4 && NV == 8 && STORE == ST_F32;
+    bool any_order = WIDE && EXACT;
+    if constexpr (WIDE && !EXACT && METRIC != M_COS) {
+        if (P.int_rows) {
+            float mn = INFINITY, mx = -INFINITY;
+            bool whole = true;
+            for (int i = lane; i < P.dim; i += 64) {
+                const float v = qv[i];
+                whole = whole && v == rintf(v);
+                mn = fminf(mn, v);
+                mx = fmaxf(mx, v);
+            }
+            for (int o = 32; o > 0; o >>= 1) {
+                mn = fminf(mn, __shfl_xor(mn, o));
+                mx = fmaxf(mx, __shfl_xor(mx, o));
+            }
+            const double a = METRIC == M_L2 ? (double)fmaxf(mx, P.row_max) - (double)fminf(mn, P.row_min)
+                                            : (double)fmaxf(fabsf(P.row_max), fabsf(P.row_min));
+            const double b = METRIC == M_L2 ? a : (double)fmaxf(fabsf(mx), fabsf(mn));
+            any_order = ballot(!whole) == 0ull && (double)P.dim * a * b < 16777216.0;
+        }
+    }
+
     bool use_cache = false;
     uint32_t epoch = 0u, cache_hits = 0u;
     DuoMail *mail = nullptr;
@@ -1064,9 +1095,9 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     // shifts and four selects and no LDS access; a merge that scattered head and new keys through LDS
     // took two dependent LDS round trips per expansion and the same work per new key.
     const auto push_head = [&](const Key &o) {
-        const uint64_t below = ballot(lt(hq, o)) & (low_bits(nq) << h);
+        const uint64_t below = ballot(lt(hq, o));  // (lanes outside [h, h + nq) hold +inf)
         const int r = __popcll(below);
-        if (h > 0) {
+        if (h > 0) [[likely]] {
             hq = ksel(in_mask(below >> 1), shl1(hq), hq);
             hq = ksel(in_mask(1ull << (h - 1 + r)), o, hq);
             --h;
@@ -1128,8 +1159,9 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     uint32_t row_id = NONE, row = 0u, ahead = 0u;
     // all lanes load (lanes past the row read its last word and are never used: a row's
     // degree is below gstride), so the load needs no lane mask and no zero fill
+    const int gshift = P.gstride == 32 ? 5 : 6;  // rows of 32 or 64 words
     const auto adj_row = [&](uint32_t v) -> uint32_t {
-        return P.graph[(size_t)v * (size_t)P.gstride + (uint32_t)min(lane, P.gstride - 1)];
+        return P.graph[((size_t)v << gshift) + (uint32_t)min(lane, P.gstride - 1)];
     };
 
     // one expansion; returns true to leave the loop
@@ -1158,6 +1190,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         // stop rule, graph.h:188: |best| == pq and best.max.d < now.d (distance only, strict)
         if (nf + nt == pq && bmax < now.dk()) [[unlikely]] return true;
         ++steps;
+        hq = ksel(in_mask(1ull << h), Key::inf(), hq);
         ++h;
         --nq;
 
@@ -1294,7 +1327,14 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
                 }
             }
         }
-        if (!cached) mine = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m, cid, qv, lenv);
+        if (!cached) {
+            if (WIDE && any_order && m <= 4) {
+                mine = eval_candidates<METRIC, EXACT, STORE, 16, 2, Key>(P, m, cid, qv, lenv);
+                have = cand_of_lane<16>() < m;
+            } else {
+                mine = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m, cid, qv, lenv);
+            }
+        }
 
         // ---- the candidates: at most T into the sorted head, above T into the bag
         const uint64_t cut = (nf + nt == pq) ? bmax : ~0ull;  // drop distance keys above cut

@@ -595,6 +595,9 @@ extern "C" int song_search_device_ex(song_index *ix, const float *d_queries, uin
     sp.dim = ix->dim;
     sp.ld = ix->ld;
     sp.gstride = ix->gstride;
+    sp.int_rows = ix->integer_valued;
+    sp.row_min = ix->vmin;
+    sp.row_max = ix->vmax;
     sp.nq = (int)nq;
     sp.pq = pq;
     sp.k = k;
