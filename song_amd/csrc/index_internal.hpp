@@ -92,6 +92,8 @@ int make_plan(const song_index *ix, bool exact, int store, int pq, int slack, in
 // LDS bytes of one query's slice in search_group (its layout: visited | queue | best | stage | cid | qv)
 size_t group_lds_bytes(bool exact, int pq, int slack, int hlog, int qld, int vis16, int lanes);
 int default_hlog(int pq);
+int roomy_hlog(const song_index *ix, bool exact, int store, int pq, int slack, uint64_t nq, int visited_bits,
+               int best_in_global);
 // Bloom filter sizing of the reference's auto_tune_bloom (auto_tune_bloom.cc:6-37, 65-86)
 void bloom_size(int pq, int *hlog32, int *k);
 SearchFn search_fn(int metric, const Plan &p, bool persistent = false);

@@ -96,7 +96,9 @@ extern "C" int song_search_device_noalloc(song_index *ix, const float *d_queries
     if (opts.slack < 0) opts.slack = 0;
     if (opts.max_steps <= 0) opts.max_steps = 1000000;
     const bool exact = opts.storage == SONG_STORE_F32 && opts.mode == SONG_MODE_EXACT;
-    int hlog = opts.hash_log2 > 0 ? opts.hash_log2 : default_hlog(pq);
+    int hlog = opts.hash_log2 > 0 ? opts.hash_log2
+                                  : roomy_hlog(ix, exact, opts.storage, pq, opts.slack, nrun, opts.visited_bits,
+                                               opts.best_in_global);
     hlog = std::max(8, std::min(hlog, 16));
     if (opts.bloom_k != 0) hlog = opts.hash_log2 > 0 ? std::min(opts.hash_log2, 15) : 0;
     Plan plan;

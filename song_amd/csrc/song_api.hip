@@ -439,6 +439,20 @@ int song::make_plan(const song_index *ix, bool exact, int store, int pq, int sla
 // whose global table overflows are re-run.
 int song::default_hlog(int pq) { return pq > 1024 ? 13 : 12; }
 
+// The default table of a call whose nq queries do not fill the device: as large as leaves all of them
+// in flight at once, up to 2^14 slots.  A fuller table costs second probes (at half load one of 31
+// neighbours finds its group full in most expansions) and, at the end, the global one; results do
+// not depend on the size.
+int song::roomy_hlog(const song_index *ix, bool exact, int store, int pq, int slack, uint64_t nq, int visited_bits,
+                     int best_in_global) {
+    int h = default_hlog(pq);
+    const uint64_t per_cu = std::max<uint64_t>(1, (nq + ix->n_cu - 1) / ix->n_cu);
+    for (Plan p; h < 14; ++h)
+        if (make_plan(ix, exact, store, pq, slack, h + 1, &p, -1, visited_bits, 0, 1, 0, 1, best_in_global, nq) != SONG_OK ||
+            ((p.lds + 15) & ~(size_t)15) * per_cu > ix->max_lds)
+            break;
+    return h;
+}
 
 SearchFn song::search_fn(int metric, const Plan &p, bool persistent) {
     if (p.duo && persistent) {
@@ -562,7 +576,9 @@ extern "C" int song_search_device_ex(song_index *ix, const float *d_queries, uin
     uint32_t *gvis = nullptr;
     int rcg = ensure_gvis(ix, stream, (size_t)std::min<uint64_t>(nrun ? nrun : 1, kChunk), &gvis);
     if (rcg != SONG_OK) return rcg;
-    int hlog = opts.hash_log2 > 0 ? opts.hash_log2 : default_hlog(pq);
+    int hlog = opts.hash_log2 > 0 ? opts.hash_log2
+                                  : roomy_hlog(ix, exact, opts.storage, pq, opts.slack, nrun, opts.visited_bits,
+                                               opts.best_in_global);
     hlog = std::max(8, std::min(hlog, 16));
     if (opts.bloom_k != 0) hlog = opts.hash_log2 > 0 ? std::min(opts.hash_log2, 15) : 0;  // 0: sized for pq
     Plan plan;
