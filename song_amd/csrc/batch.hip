@@ -113,7 +113,9 @@ struct song_batch {
     std::vector<Cached> graphs;
 };
 
-static int default_tier_hlog(int pq) { return default_hlog(pq); }
+// A tier of two waves per query is latency-bound and its registers admit 6-8 groups per CU, which
+// leaves LDS for a table twice as large: its long searches then stay out of the global table.
+static int default_tier_hlog(const song_tier &t) { return default_hlog(t.pq_max) + (t.waves_per_query == 2 ? 1 : 0); }
 
 extern "C" void song_batch_config_default(song_batch_config *c, int pq_max) {
     memset(c, 0, sizeof(*c));
@@ -244,12 +246,12 @@ extern "C" int song_batch_create(song_index *ix, const song_batch_config *cfg, u
     int top_hlog = 0;
     for (int t = 0; t < c.n_tiers; ++t)
         if (c.tier[t].bloom_k == 0)
-            top_hlog = std::max(top_hlog, c.tier[t].hash_log2 ? c.tier[t].hash_log2 : default_tier_hlog(c.tier[t].pq_max));
-    if (top_hlog == 0) top_hlog = default_tier_hlog(pq_top);
+            top_hlog = std::max(top_hlog, c.tier[t].hash_log2 ? c.tier[t].hash_log2 : default_tier_hlog(c.tier[t]));
+    if (top_hlog == 0) top_hlog = default_hlog(pq_top);
     for (int t = 0; t <= c.n_tiers; ++t) {
         const bool is_retry = t == c.n_tiers;
         const song_tier &ti = is_retry ? rt : c.tier[t];
-        int hlog = ti.hash_log2 ? ti.hash_log2 : (ti.bloom_k ? 0 : default_tier_hlog(ti.pq_max));
+        int hlog = ti.hash_log2 ? ti.hash_log2 : (ti.bloom_k ? 0 : default_tier_hlog(ti));
         if (is_retry && !ti.hash_log2) hlog = std::min(16, top_hlog + 2);
         Launch L;
         L.pq_max = ti.pq_max;

@@ -376,7 +376,7 @@ __device__ __forceinline__ bool vis16_test(const uint32_t *vis, int gbits, int i
     return false;
 }
 
-// insert into this query's global spill table (same scheme, device-scope CAS)
+// insert into a query's global spill table, one slot per probe (sub-groups of a wave, device-scope CAS)
 __device__ __forceinline__ bool gvis_insert(uint32_t *g, uint32_t mask, int hlog, uint32_t id) {
     const uint32_t key = id + 1u;
     uint32_t s = (id * 0x9E3779B1u) >> (32 - hlog);
@@ -386,6 +386,43 @@ __device__ __forceinline__ bool gvis_insert(uint32_t *g, uint32_t mask, int hlog
         if (old == key) return false;
         s = (s + 1u) & mask;
     }
+}
+
+// The same table for a whole wave that owns it, without atomics: lanes with `want` insert their id and
+// learn whether it was absent.  A lane reads its home group of four slots (16 bytes, one round trip);
+// an id with a free slot there claims it through one LDS word per 64th of the slots (arb, 64 u32),
+// so that lanes after the same slot -- the same id included -- take turns, and stores it without
+// waiting.  An atomic compare-and-swap per probe, the other form, is a round trip to L2 for every
+// lane and probe: the searches that outgrow their LDS table (the longest of a launch) spent most of
+// their time on it.
+__device__ __forceinline__ bool gvis_claim(uint32_t *g, int hlog, uint32_t id, bool want, uint32_t *arb) {
+    const uint32_t key = id + 1u, gmask = (1u << (hlog - 2)) - 1u;
+    const int lane = lane_id();
+    uint32_t grp = (id * 0x9E3779B1u) >> (34 - hlog);
+    bool fresh = false;
+    bag_fence();
+    while (ballot(want) != 0ull) {
+        if (want) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(g + (grp << 2));
+            const uint32_t e = v.x == 0u ? 0u : v.y == 0u ? 1u : v.z == 0u ? 2u : v.w == 0u ? 3u : 4u;
+            if (v.x == key || v.y == key || v.z == key || v.w == key) {
+                want = false;
+            } else if (e == 4u) {
+                grp = (grp + 1u) & gmask;
+            } else {
+                const uint32_t slot = (grp << 2) + e;
+                arb[slot & 63u] = (uint32_t)lane;
+                lds_fence();
+                if (arb[slot & 63u] == (uint32_t)lane) {
+                    g[slot] = key;
+                    fresh = true;
+                    want = false;
+                }
+            }
+        }
+        if (ballot(want) != 0ull) bag_fence();  // the stores above, before the groups are read again
+    }
+    return fresh;
 }
 
 // Blocked Bloom filter (the reference's BlockedBloomFilter, blocked_bloomfilter.h:9-82, with
@@ -1072,10 +1109,10 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         vmode = V_SPILL;
         vstop = ~0u;
         gv = P.gvis + (size_t)slot_q * (1u << P.ghlog);
-        for (uint32_t i = (uint32_t)rare_lane(); i < (1u << P.ghlog); i += 64) gv[i] = 0u;
-        __threadfence_block();
+        for (uint32_t i = (uint32_t)rare_lane(); i < (1u << P.ghlog) / 4; i += 64)
+            reinterpret_cast<uint4 *>(gv)[i] = make_uint4(0u, 0u, 0u, 0u);
     };
-    const uint32_t GH = 1u << P.ghlog, gmask = GH - 1u, glimit = (GH >> 2) * 3u;
+    const uint32_t glimit = ((1u << P.ghlog) >> 2) * 3u;
     int h = 0, nq = 0;
     // The best list (the pq smallest expanded keys): its largest nt <= 64 entries, the tail, ascending in
     // lanes [0, nt) of a register (+inf above), the other nf, the front, in memory in any order.  Only the
@@ -1287,7 +1324,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
                     return true;
                 }
                 to_spill();
-                if (vovf) fresh = gvis_insert(gv, gmask, P.ghlog, r);
+                if (gvis_claim(gv, P.ghlog, r, vovf, cid)) fresh = true;
             }
         } else if (vmode == V_32) {
             if (in_mask(nb)) fresh = vis_insert(vis, hmask, P.hlog, r);
@@ -1296,7 +1333,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         } else {
             bool in_lds = true;
             if (in_mask(nb)) in_lds = P.vis16 ? vis16_test(vis, gbits, P.idbits, r) : vis_test(vis, hmask, P.hlog, r);
-            if (!in_lds) fresh = gvis_insert(gv, gmask, P.ghlog, r);
+            fresh = gvis_claim(gv, P.ghlog, r, !in_lds, cid);
         }
         const uint64_t fm = ballot(fresh);
         const int m = __popcll(fm);
