@@ -426,6 +426,7 @@ static int enqueue(song_batch *b, const RunArgs &a, hipStream_t st) {
         p.gbag_stride = L.bag_stride;
         p.wave_lds = (uint32_t)L.wave_lds;
         p.vis16 = L.plan.vis16;
+        p.seq_stage = L.plan.seq_stage;
         p.bloom_k = L.plan.bloom_k;
         p.multiprobe = L.multiprobe;
         p.idbits = ix->idbits;

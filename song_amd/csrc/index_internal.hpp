@@ -72,6 +72,7 @@ struct Plan {
     int duo;     // two waves per query (search_duo: search wave + helper wave)
     int pq;      // budget the layout is sized for
     int bglob;   // search_query's best-list front in global memory, after the slot's bag
+    int seq_stage; // exact mode on wide rows: SEQ_STAGE floats of LDS after the query
     size_t lds;  // LDS bytes of one wave (lanes 64) or of one query's slice (lanes 16 / 32)
 };
 

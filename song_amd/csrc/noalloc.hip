@@ -172,6 +172,7 @@ extern "C" int song_search_device_noalloc(song_index *ix, const float *d_queries
     sp.ghlog = kGhlog;
     sp.wave_lds = (uint32_t)wave_lds;
     sp.vis16 = plan.vis16;
+    sp.seq_stage = plan.seq_stage;
     sp.bloom_k = plan.bloom_k;
     sp.idbits = ix->idbits;
     sp.data_lp = ix->d_lp[plan.store];

@@ -25,6 +25,7 @@
 //              bglob, where the front lives in the wave slot's global region
 //   cid      : 256 u32   candidate ids of the current expansion / radix-select bins
 //   qv       : qld f32   the query, zero-padded to a multiple of 16
+//   stage    : products of the exact sums done again (wide rows in exact mode, seq_stage)
 // The queue head is one key per lane in registers, ascending over lanes [h, h + nq), nq <= 64,
 // +inf in the others.
 // The bag (qcap = pq + slack + 128 keys, unsorted, first bn live) is in global memory, one
@@ -107,6 +108,7 @@ struct SearchParams {
                             // bloom_k bits per id in one word (approximate: false positives skip vertices)
     int multiprobe;         // several-queries-per-wave kernel: expansions per step (1, or 2: the next
                             // queue head too; approximate)
+    int seq_stage;          // 1: the slice has SEQ_STAGE floats after the query
     int int_rows;           // 1: every row value is an integer, in [row_min, row_max]
     float row_min, row_max;
 };
@@ -478,58 +480,82 @@ __device__ __forceinline__ float finish_f32(float s, float lena, float lenv) {
 
 // One lane, sequential over the dimensions in the CPU's order (exact fallback).  Both operands are
 // read in 16-byte units; the row and the query are zero past dim, and a zero product leaves the sum
-// as it is.  What bounds it is the chain of double additions, so everything else is kept off it: row
-// units are loaded in two alternating blocks of AHEAD, one in flight while the other is used, and a
-// block's query reads and products come before its additions.  Wide rows take 8 units a block;
-// narrow ones, whose sums are short and seldom need this, 1, which keeps the registers (and so the
-// waves per SIMD) of their kernels.  1,000 queries on 960 dimensions: 10.36 -> 9.47 ms; with 8 units for
-// rows of 16 dimensions too, 5,000 cosine queries took 988 instead of 752 us (two waves per SIMD).
-template <int METRIC, int AHEAD = 1>
+// as it is.
+template <int METRIC> __device__ __forceinline__ float product(float x, float q) {
+    if (METRIC == M_L2) {
+        const float d = x - q;
+        return d * d;
+    }
+    return x * q;
+}
+template <int METRIC>
 __device__ double seq_sum(const float *row, const float *qv, int dim) {
     const float4 *r4 = reinterpret_cast<const float4 *>(row);
     const float4 *q4 = reinterpret_cast<const float4 *>(qv);
     const int nu = (dim + 3) >> 2;
     double s = 0.0;
-    const auto prod = [](float x, float q) {
-        if (METRIC == M_L2) {
-            const float d = x - q;
-            return d * d;
-        }
-        return x * q;
-    };
-    float4 xa[AHEAD], xb[AHEAD];
-    const auto load = [&](float4 (&x)[AHEAD], int j) {
-#pragma unroll
-        for (int t = 0; t < AHEAD; ++t) x[t] = r4[min(j + t, nu - 1)];
-    };
-    const auto take = [&](float4 (&x)[AHEAD], int j) {
-        float4 q[AHEAD];
-#pragma unroll
-        for (int t = 0; t < AHEAD; ++t) q[t] = q4[min(j + t, nu - 1)];
-#pragma unroll
-        for (int t = 0; t < AHEAD; ++t) {
-            // a unit past the row contributes zeros
-            const bool in = j + t < nu;
-            x[t].x = in ? prod(x[t].x, q[t].x) : 0.0f;
-            x[t].y = in ? prod(x[t].y, q[t].y) : 0.0f;
-            x[t].z = in ? prod(x[t].z, q[t].z) : 0.0f;
-            x[t].w = in ? prod(x[t].w, q[t].w) : 0.0f;
-        }
-#pragma unroll
-        for (int t = 0; t < AHEAD; ++t) {
-            s += (double)x[t].x;
-            s += (double)x[t].y;
-            s += (double)x[t].z;
-            s += (double)x[t].w;
-        }
-    };
-    load(xa, 0);
-    for (int j = 0; j < nu; j += 2 * AHEAD) {
-        load(xb, j + AHEAD);
-        take(xa, j);
-        load(xa, j + 2 * AHEAD);
-        take(xb, j + AHEAD);
+    float4 nx = r4[0];
+    for (int j = 0; j < nu; ++j) {
+        const float4 x = nx, q = q4[j];
+        nx = r4[min(j + 1, nu - 1)];
+        s += (double)product<METRIC>(x.x, q.x);
+        s += (double)product<METRIC>(x.y, q.y);
+        s += (double)product<METRIC>(x.z, q.z);
+        s += (double)product<METRIC>(x.w, q.w);
     }
+    return s;
+}
+
+// The same sums of 16 rows by a whole wave: lanes 4c .. 4c + 3 give row c's address, lane c returns
+// its sum (c < 16).  What bounds the sum is its chain of double additions, one lane per row; the
+// products of 64 dimensions at a time are made by all 64 lanes (4 per row, the next 64 dimensions'
+// loads in flight) and handed over through LDS, so that the chain is a conversion and an addition per
+// dimension.  With the loads, differences and products in the chain's own lane, 1,000 queries on rows of
+// 960 dimensions took 9.31 ms and take 6.55 ms with the chain alone (242 -> 139 vector registers).
+constexpr int SEQ_LD = 17;                      // float4s of a staged row: 16 and one to spread the banks
+constexpr int SEQ_STAGE = 16 * SEQ_LD * 4;      // floats
+template <int METRIC>
+__device__ __forceinline__ double seq_sum16(const float *row, const float *qv, int dim, float *stage) {
+    const int lane = lane_id(), c = lane >> 2, sub = lane & 3;
+    const float4 *r4 = reinterpret_cast<const float4 *>(row);
+    const float4 *q4 = reinterpret_cast<const float4 *>(qv);
+    float4 *st = reinterpret_cast<float4 *>(stage);
+    const int nu = (dim + 3) >> 2;
+    double s = 0.0;
+    float4 x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = r4[min(sub + 4 * i, nu - 1)];
+    for (int u0 = 0; u0 < nu; u0 += 16) {
+        lds_fence();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int u = u0 + sub + 4 * i;
+            const float4 q = q4[min(u, nu - 1)];
+            const bool in = u < nu;
+            st[c * SEQ_LD + sub + 4 * i] =
+                make_float4(in ? product<METRIC>(x[i].x, q.x) : 0.0f, in ? product<METRIC>(x[i].y, q.y) : 0.0f,
+                            in ? product<METRIC>(x[i].z, q.z) : 0.0f, in ? product<METRIC>(x[i].w, q.w) : 0.0f);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = r4[min(u0 + 16 + sub + 4 * i, nu - 1)];
+        lds_fence();
+        if (lane < 16) {
+#pragma unroll
+            for (int h = 0; h < 16; h += 8) {
+                float4 p[8];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) p[t] = st[lane * SEQ_LD + h + t];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    s += (double)p[t].x;
+                    s += (double)p[t].y;
+                    s += (double)p[t].z;
+                    s += (double)p[t].w;
+                }
+            }
+        }
+    }
+    lds_fence();
     return s;
 }
 
@@ -617,9 +643,10 @@ template <int SUB> __device__ __forceinline__ int cand_of_lane() {
 // line (units past the row are clamped and their sum dropped by a select), so that the query's LDS
 // reads and the row loads are all in flight together; with a branch per unit each unit waited for
 // its own LDS reads.
+// stage: LDS for the exact sums done again (SEQ_STAGE floats), or null.
 template <int METRIC, bool EXACT, int STORE, int SUB, int NVU, class Key>
 __device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, const uint32_t *cid, const float *qv,
-                                               float lenv) {
+                                               float lenv, float *stage = nullptr) {
     constexpr int EPU = Store<STORE>::EPU;
     const int lane = lane_id();
     constexpr int G = 64 / SUB;
@@ -731,12 +758,29 @@ __device__ __forceinline__ Key eval_candidates(const SearchParams &P, int m, con
         }
     }
     if constexpr (EXACT) {
-        // sequential re-evaluation in the CPU's order, one lane per flagged candidate
-        if (redo) {
-            const uint32_t id = mine.id();
-            const float lena = (METRIC == M_COS) ? P.norms[id] : 0.0f;
-            const double s = seq_sum<METRIC, (SUB * NVU > 64 ? 8 : 1)>(P.data + (size_t)id * (size_t)P.ld, qv, P.dim);
-            mine = Key::make_d(finish_exact<METRIC>(s, lena, lenv), id);
+        // sequential re-evaluation in the CPU's order of the flagged candidates: up to 16 at a time
+        // through the stage, or one lane each
+        const uint64_t todo = ballot(redo);
+        if (todo != 0ull) {
+            double s = 0.0;
+            if (SUB * NVU > 64 && stage) {
+                const int rank = lanes_below(todo), n = __popcll(todo);
+                for (int c0 = 0; c0 < n; c0 += 16) {
+                    const bool now = redo && rank >= c0 && rank < c0 + 16;
+                    if (now) reinterpret_cast<uint32_t *>(stage)[rank - c0] = mine.id();
+                    lds_fence();
+                    const uint32_t id = reinterpret_cast<const uint32_t *>(stage)[min(lane >> 2, n - c0 - 1)];
+                    const double t = seq_sum16<METRIC>(P.data + (size_t)id * (size_t)P.ld, qv, P.dim, stage);
+                    const double got = __shfl(t, (rank - c0) & 63);
+                    if (now) s = got;
+                }
+            } else if (redo) {
+                s = seq_sum<METRIC>(P.data + (size_t)mine.id() * (size_t)P.ld, qv, P.dim);
+            }
+            if (redo) {
+                const float lena = (METRIC == M_COS) ? P.norms[mine.id()] : 0.0f;
+                mine = Key::make_d(finish_exact<METRIC>(s, lena, lenv), mine.id());
+            }
         }
     }
     return mine;
@@ -1003,12 +1047,14 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
     uint32_t *cid = reinterpret_cast<uint32_t *>(B + (bglob ? 0 : ((P.pq + 1) & ~1)));  // 256 u32
     float *qv = reinterpret_cast<float *>(cid + 256);
     // bag, qcap keys: global memory (one region per slot), or this wave's LDS after the query
-    Key *Bg = BAGL ? reinterpret_cast<Key *>(qv + P.qld)
+    float *stage = (EXACT && P.seq_stage) ? qv + P.qld : nullptr;  // SEQ_STAGE floats
+    float *qv_end = qv + P.qld + ((EXACT && P.seq_stage) ? SEQ_STAGE : 0);
+    Key *Bg = BAGL ? reinterpret_cast<Key *>(qv_end)
                    : reinterpret_cast<Key *>(P.gbag + (size_t)slot_q * P.gbag_stride);
     // the layout must fit the slice and the bag the launch allocated: otherwise flag the query
     // and touch neither (a host / kernel mismatch becomes an error, not out-of-range accesses)
     const unsigned char *lds_end = BAGL ? reinterpret_cast<unsigned char *>(Bg + P.qcap)
-                                        : reinterpret_cast<unsigned char *>(qv + P.qld);
+                                        : reinterpret_cast<unsigned char *>(qv_end);
     const size_t gneed = bglob ? bag_bytes<Key>(P.qcap) + (size_t)P.pq * sizeof(Key) : (size_t)P.qcap * sizeof(Key);
     if (lds_end - smem > (ptrdiff_t)P.wave_lds ||
         (!BAGL && (!P.gbag || gneed > P.gbag_stride))) {
@@ -1179,7 +1225,7 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         if (fresh) cid[lanes_below(fm)] = sid;
         nvis = (uint32_t)m0;
         lds_fence();
-        const Key k0 = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m0, cid, qv, lenv);
+        const Key k0 = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m0, cid, qv, lenv, stage);
         for (uint64_t bits = ballot(cand_of_lane<SUB>() < m0); bits; bits &= bits - 1) push_head(k0.rl(__builtin_ctzll(bits)));
         lds_fence();
     }
@@ -1366,10 +1412,10 @@ __device__ __forceinline__ void search_query(const SearchParams &P, const int qi
         }
         if (!cached) {
             if (WIDE && any_order && m <= 4) {
-                mine = eval_candidates<METRIC, EXACT, STORE, 16, 2, Key>(P, m, cid, qv, lenv);
+                mine = eval_candidates<METRIC, EXACT, STORE, 16, 2, Key>(P, m, cid, qv, lenv, stage);
                 have = cand_of_lane<16>() < m;
             } else {
-                mine = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m, cid, qv, lenv);
+                mine = eval_candidates<METRIC, EXACT, STORE, SUB, NV, Key>(P, m, cid, qv, lenv, stage);
             }
         }
 

@@ -404,7 +404,8 @@ extern "C" int song_index_integer_valued(const song_index *ix) { return ix ? ix-
 
 // must match the per-wave layout of search_query: visited (2^hlog slots of 4 or, compact, 2
 // bytes) | best (pq rounded to even; not with bglob) | 256
-// candidate ids / radix bins | query (the head is in registers, the bag in global memory)
+// candidate ids / radix bins | query (the head is in registers, the bag in global memory) | with
+// seq_stage (make_plan adds it) the exact sums' stage
 size_t song::lds_bytes(bool exact, int pq, int qcap, int hlog, int qld, int vis16, int bloom_k, int bag_lds,
                        int bglob) {
     size_t key = exact ? 16 : 8;
@@ -502,6 +503,7 @@ int song::make_plan(const song_index *ix, bool exact, int store, int pq, int sla
     const int lob = ix->idbits - (hlog - 3);
     p->vis16 = (bloom_k == 0 && visited_bits != 32 && hlog >= 4 && lob >= 0 && lob <= 13) ? 1 : 0;
     p->bglob = best_in_global == 1 ? 1 : 0;
+    p->seq_stage = 0;
     if (best_in_global < 0 && bglob_ok) {
         const size_t lds_front = (lds_bytes(p->exact, pq, p->qcap, hlog, p->qld, p->vis16, bloom_k, 0, 0) + 15) & ~15;
         const uint64_t per_cu = std::max<uint64_t>(1, ix->max_lds / lds_front);
@@ -512,6 +514,13 @@ int song::make_plan(const song_index *ix, bool exact, int store, int pq, int sla
         p->lds = group_lds_bytes(p->exact, pq, slack, hlog, p->qld, p->vis16, p->lanes);
     } else {
         p->lds = lds_bytes(p->exact, pq, p->qcap, hlog, p->qld, p->vis16, bloom_k, p->bag_lds, p->bglob);
+        // exact sums of wide rows (the shapes that share a row among 16 or more lanes) are done again
+        // through LDS, where the slice has room for it
+        const size_t more = SEQ_STAGE * sizeof(float);
+        if (p->exact && p->shape >= 3 && p->lds + more <= ix->max_lds) {
+            p->seq_stage = 1;
+            p->lds += more;
+        }
     }
     if (p->lds > ix->max_lds)
         return fail(SONG_E_OVERFLOW, "search needs %zu bytes of LDS per query (> %zu)", p->lds, ix->max_lds);
@@ -577,6 +586,7 @@ static int launch(song_index *ix, const Plan &p, SearchParams sp, unsigned count
     sp.qld = p.qld;
     sp.wave_lds = (uint32_t)p.lds;
     sp.vis16 = p.vis16;
+    sp.seq_stage = p.seq_stage;
     sp.bloom_k = p.bloom_k;
     sp.idbits = ix->idbits;
     sp.data_lp = ix->d_lp[p.store];
