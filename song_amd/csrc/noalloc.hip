@@ -98,7 +98,7 @@ extern "C" int song_search_device_noalloc(song_index *ix, const float *d_queries
     const bool exact = opts.storage == SONG_STORE_F32 && opts.mode == SONG_MODE_EXACT;
     int hlog = opts.hash_log2 > 0 ? opts.hash_log2
                                   : roomy_hlog(ix, exact, opts.storage, pq, opts.slack, nrun, opts.visited_bits,
-                                               opts.best_in_global);
+                                               opts.best_in_global, true);
     hlog = std::max(8, std::min(hlog, 16));
     if (opts.bloom_k != 0) hlog = opts.hash_log2 > 0 ? std::min(opts.hash_log2, 15) : 0;
     Plan plan;

@@ -505,7 +505,7 @@ int song::make_plan(const song_index *ix, bool exact, int store, int pq, int sla
     p->bglob = best_in_global == 1 ? 1 : 0;
     p->seq_stage = 0;
     if (best_in_global < 0 && bglob_ok) {
-        const size_t lds_front = (lds_bytes(p->exact, pq, p->qcap, hlog, p->qld, p->vis16, bloom_k, 0, 0) + 15) & ~15;
+        const size_t lds_front = lds_granted(lds_bytes(p->exact, pq, p->qcap, hlog, p->qld, p->vis16, bloom_k, 0, 0));
         const uint64_t per_cu = std::max<uint64_t>(1, ix->max_lds / lds_front);
         p->bglob = (nq_hint == 0 || nq_hint > per_cu * (uint64_t)ix->n_cu) ? 1 : 0;
     }
@@ -533,18 +533,47 @@ int song::make_plan(const song_index *ix, bool exact, int store, int pq, int sla
 // whose global table overflows are re-run.
 int song::default_hlog(int pq) { return pq > 1024 ? 13 : 12; }
 
-// The default table of a call whose nq queries do not fill the device: as large as leaves all of them
-// in flight at once, up to 2^14 slots.  A fuller table costs second probes (at half load one of 31
-// neighbours finds its group full in most expansions) and, at the end, the global one; results do
-// not depend on the size.
+// waves of a plan that one CU holds, by its LDS and by the kernel's registers; 0 = unknown
+static int waves_per_cu(const song_index *ix, const Plan &p, bool persistent) {
+    const SearchFn fn = search_fn(ix->metric, p, persistent);
+    const size_t lds = (p.lds + 15) & ~(size_t)15;
+    int n = 0;
+    if (!fn || lds > 65536 ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)fn, 64, lds) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return (int)std::min<size_t>((size_t)n, ix->max_lds / lds_granted(lds));
+}
+
+// The default table of a plain or no-allocation call.  Results do not depend on the size.
+//
+// Where its nq queries leave LDS free: as large as leaves all of them in flight at once, up to 2^14
+// slots.  A fuller table costs second probes (at half load one of 31 neighbours finds its group full in
+// most expansions) and, at the end, the global one.
+//
+// Where they do not fit at once: half the table if a CU then holds at least a sixth more waves and these
+// take them in fewer rounds.  The kernels of rows up to 32 floats, and of narrow 16- and 8-bit rows,
+// leave registers for 20 to 24 waves where 2^12 slots leave LDS for 16.  Up to 100k rows and pq 128 few
+// searches outgrow 2^11 slots: cosine 15k x 16, 5000 queries at pq 100, exact 668 -> 574 us; 100k x 32
+// uniform rows, 9000 queries at pq 100, 935 -> 877 us, bf16 943 -> 892.  As many rounds as before lose
+// (the same set, 7000 queries: 778 -> 811), and so do a few more waves over many rounds (100k x 96 in
+// bf16, 14 -> 16 waves, 30,000 queries at pq 100: 3866 -> 4080), larger budgets (50k x 24, 20,000 queries
+// at pq 256: 3499 -> 3689), larger sets (1M x 32, 4500 queries at pq 100: 929 -> 1138) and 2^10 slots.
 int song::roomy_hlog(const song_index *ix, bool exact, int store, int pq, int slack, uint64_t nq, int visited_bits,
-                     int best_in_global) {
+                     int best_in_global, bool persistent) {
     int h = default_hlog(pq);
     const uint64_t per_cu = std::max<uint64_t>(1, (nq + ix->n_cu - 1) / ix->n_cu);
-    for (Plan p; h < 14; ++h)
-        if (make_plan(ix, exact, store, pq, slack, h + 1, &p, -1, visited_bits, 0, 1, 0, 1, best_in_global, nq) != SONG_OK ||
-            ((p.lds + 15) & ~(size_t)15) * per_cu > ix->max_lds)
-            break;
+    auto plan = [&](int hlog, Plan *p) {
+        return make_plan(ix, exact, store, pq, slack, hlog, p, -1, visited_bits, 0, 1, 0, 1, best_in_global, nq) == SONG_OK;
+    };
+    Plan p;
+    while (h < 14 && plan(h + 1, &p) && lds_granted(p.lds) * per_cu <= ix->max_lds) ++h;
+    Plan half;
+    if (h == default_hlog(pq) && pq <= 128 && ix->n <= 100000 && plan(h, &p) && plan(h - 1, &half)) {
+        const uint64_t now = waves_per_cu(ix, p, persistent), more = waves_per_cu(ix, half, persistent);
+        if (now > 0 && 6 * more >= 7 * now && (per_cu + more - 1) / more < (per_cu + now - 1) / now) --h;
+    }
     return h;
 }
 
@@ -673,7 +702,7 @@ extern "C" int song_search_device_ex(song_index *ix, const float *d_queries, uin
     if (rcg != SONG_OK) return rcg;
     int hlog = opts.hash_log2 > 0 ? opts.hash_log2
                                   : roomy_hlog(ix, exact, opts.storage, pq, opts.slack, nrun, opts.visited_bits,
-                                               opts.best_in_global);
+                                               opts.best_in_global, false);
     hlog = std::max(8, std::min(hlog, 16));
     if (opts.bloom_k != 0) hlog = opts.hash_log2 > 0 ? std::min(opts.hash_log2, 15) : 0;  // 0: sized for pq
     Plan plan;
